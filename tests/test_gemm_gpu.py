@@ -219,3 +219,64 @@ def test_gemm_saturation_and_nonfinite(gpu, oracle):
     assert rel_err(Y[ok], ref) <= TOL
     assert np.all(np.isnan(Y[5]))
     assert np.all(~np.isfinite(Y[6]))
+
+
+# One shape per K-split tile (32 x 32, 32 x 64, 64 x 64, 64 x 128, 64 x 256,
+# 96 x 128, 96 x 256, 128 x 128, 128 x 256 tokens x weight rows) at sizes off
+# the tile edges, then the edges themselves: one weight subtile, one K group
+# (fewer than the block's parts), parts of unequal length (G = 13, 29), a
+# token over and under a tile.
+@pytest.mark.parametrize("T,N,K,zeros", [(21, 2048, 2048, True), (35, 5120, 2048, False), (43, 8704, 2048, True),
+                                         (95, 12288, 2048, True), (1567, 5120, 1664, True), (502, 5120, 2048, False),
+                                         (1074, 4096, 2048, True), (673, 4144, 3712, True), (1788, 8176, 1920, False),
+                                         (1, 16, 128, True), (33, 48, 256, False), (32, 272, 1664, True),
+                                         (65, 2048, 3712, True), (129, 1040, 640, False)])
+def test_gemm_ksplit_shapes(gpu, oracle, T, N, K, zeros):
+    """Strided fp16 rows and a strided output: fp32 rows within the tolerance
+    of the oracle, nothing written past a row's N columns, and fp16 and bf16
+    rows the roundings of the fp32 ones bit for bit."""
+    import torch
+    print(f"gemm K-split T={T} N={N} K={K} zeros={zeros}", flush=True)
+    W, S, Z = synth.q4_weights(T + N, f"ks{N}x{K}", N, K, zeros)
+    _, xf = synth.acts(T + K, f"ksx{T}x{K}", T, K)
+    x16 = xf.astype(np.float16)
+    dW, dS, dZ = qwq4.tile(to_dev(W, gpu), to_dev(S, gpu), to_dev(Z, gpu) if zeros else None, N, K)
+    X = torch.full((T, K + 8), float("nan"), dtype=torch.float16, device=gpu)[:, :K]
+    X.copy_(torch.from_numpy(x16))
+    ys = {}
+    for dt in (torch.float32, torch.float16, torch.bfloat16):
+        Y = torch.full((T, N + 16), 7.0, dtype=dt, device=gpu)
+        qwq4.gemm(dW, dS, dZ, X, N, K, Y=Y)
+        assert bool((Y[:, N:] == 7.0).all())
+        ys[dt] = Y[:, :N]
+    y32 = ys[torch.float32]
+    assert torch.equal(ys[torch.bfloat16], y32.to(torch.bfloat16))
+    assert np.array_equal(host(ys[torch.float16].contiguous()).view(np.uint16), _f16_sat(host(y32.contiguous())).view(np.uint16))
+    r = np.random.default_rng(T)
+    toks = np.sort(np.unique(np.r_[0, T - 1, r.choice(T, min(T, 24), replace=False)]))
+    rows = np.sort(np.unique(np.r_[0, N - 1, r.choice(N, min(N, 256), replace=False)]))
+    ref = oracle.q4_linear(W[rows], S[rows], Z[rows] if zeros else None, len(rows), K, x16.astype(np.float32)[toks])
+    assert rel_err(host(y32.contiguous())[np.ix_(toks, rows)], ref) <= TOL
+
+
+def test_gemm_ksplit_nonfinite(gpu, oracle):
+    """Infinities and NaN in a row of a short chunk: what the plain product
+    gives (an infinity times a zero weight is NaN, times any other an infinity
+    of that sign), other rows untouched."""
+    import torch
+    T, N, K = 40, 512, 1280
+    W, S, Z = synth.q4_weights(58, "ksinf", N, K)
+    _, xf = synth.acts(58, "ksinfx", T, K)
+    x = xf.astype(np.float16)
+    x[3, 700] = np.inf
+    x[7, 1279] = -np.inf
+    x[9, 0] = np.nan
+    dW, dS, dZ = qwq4.tile(to_dev(W, gpu), to_dev(S, gpu), to_dev(Z, gpu), N, K)
+    Y = host(qwq4.gemm(dW, dS, dZ, torch.from_numpy(x).to(gpu), N, K))
+    w = oracle.q4_dequant(W, S, Z, N, K)
+    with np.errstate(invalid="ignore"):
+        assert np.array_equal(Y[3], np.where(w[:, 700] == 0, np.nan, np.inf * w[:, 700]).astype(np.float32), equal_nan=True)
+        assert np.array_equal(Y[7], np.where(w[:, 1279] == 0, np.nan, -np.inf * w[:, 1279]).astype(np.float32), equal_nan=True)
+    assert np.all(np.isnan(Y[9]))
+    ok = [t for t in range(T) if t not in (3, 7, 9)]
+    assert rel_err(Y[ok], oracle.q4_linear(W, S, Z, N, K, x[ok].astype(np.float32))) <= TOL

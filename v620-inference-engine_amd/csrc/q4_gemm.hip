@@ -12,7 +12,8 @@
 // ~1.4e-3 of max|y| (close to the 2e-3 bar); fp16 costs ~2e-4.
 //
 // Schedule: q4_gemm_core.cuh (block tile 256 or 128 tokens x 256 weight
-// rows, 8 waves, LDS double-buffered K stages of 64). Blocks take their tiles
+// rows, 8 waves, LDS double-buffered K stages of 64), or for chunks with too
+// few such tiles the K-split tiles of q4_gemm_ksplit.cuh. Blocks take their tiles
 // in an XCD-aware order; the epilogue goes through LDS so that stores are
 // 16 bytes per lane.
 #include "q4_gemm_core.cuh"
@@ -142,11 +143,7 @@ static void launch_gemm_mixed(const GemmArgs &a, const uint16_t *Xh, int lda, in
 }
 
 template <bool HAS_Z, int YT>
-static void launch_gemm_m(const GemmArgs &a, const uint16_t *Xh, int lda, hipStream_t s) {
-    int cus = 0, dev = 0;
-    (void)hipGetDevice(&dev);
-    (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
-    if (cus < 1) cus = 256;
+static void launch_gemm_m(const GemmArgs &a, const uint16_t *Xh, int lda, int cus, hipStream_t s) {
     auto whole = [&](int64_t nb) {
         const double rounds = double(nb) / cus;
         return rounds >= 4.0 || (rounds >= 1.0 && rounds - double(int64_t(rounds)) < 0.01);
@@ -170,14 +167,19 @@ void launch_gemm(const GemmArgs &a, hipStream_t s) {
         Xh = w;
         lda = a.K;
     }
+    int cus = 0, dev = 0;
+    (void)hipGetDevice(&dev);
+    (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
+    if (cus < 1) cus = 256;
+    if (launch_gemm_ksplit(a, Xh, lda, cus, s)) return;
     if (a.Z) {
-        if (a.y_type == 1) launch_gemm_m<true, 1>(a, Xh, lda, s);
-        else if (a.y_type == 2) launch_gemm_m<true, 2>(a, Xh, lda, s);
-        else launch_gemm_m<true, 0>(a, Xh, lda, s);
+        if (a.y_type == 1) launch_gemm_m<true, 1>(a, Xh, lda, cus, s);
+        else if (a.y_type == 2) launch_gemm_m<true, 2>(a, Xh, lda, cus, s);
+        else launch_gemm_m<true, 0>(a, Xh, lda, cus, s);
     } else {
-        if (a.y_type == 1) launch_gemm_m<false, 1>(a, Xh, lda, s);
-        else if (a.y_type == 2) launch_gemm_m<false, 2>(a, Xh, lda, s);
-        else launch_gemm_m<false, 0>(a, Xh, lda, s);
+        if (a.y_type == 1) launch_gemm_m<false, 1>(a, Xh, lda, cus, s);
+        else if (a.y_type == 2) launch_gemm_m<false, 2>(a, Xh, lda, cus, s);
+        else launch_gemm_m<false, 0>(a, Xh, lda, cus, s);
     }
 }
 

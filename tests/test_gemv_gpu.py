@@ -181,3 +181,22 @@ def test_read_probe_runs():
     torch.cuda.synchronize()
     with pytest.raises(RuntimeError):
         qwq4.read_probe(t[:1000])
+
+
+# K whose group count leaves the last wave a part of its chunk (5, 13, 29, 43
+# groups), more than 16 chunks (86 groups: two passes per wave), staged rows
+# that end inside a wave instruction (K / 8 not a multiple of 64) and rows
+# shorter than one (K = 384); N giving one and several subtiles per block.
+@pytest.mark.parametrize("K", [384, 640, 1664, 3712, 5504, 11008])
+@pytest.mark.parametrize("N,M,f16", [(16, 1, False), (1040, 5, True), (4112, 3, False), (528, 17, False), (4128, 16, True)])
+def test_gemv_ragged_k(gpu, oracle, N, K, M, f16):
+    import torch
+    print(f"gemv ragged N={N} K={K} M={M} f16={f16}", flush=True)
+    W, S, Z = synth.q4_weights(K + N, f"rk{N}x{K}", N, K)
+    _, xf = synth.acts(K + M, f"rkx{M}x{K}", M, K)
+    dW, dS, dZ = qwq4.tile(to_dev(W, gpu), to_dev(S, gpu), to_dev(Z, gpu), N, K)
+    x = torch.from_numpy(xf).to(gpu).to(torch.float16 if f16 else torch.bfloat16)
+    xf = host(x.float())
+    y = torch.full((M, N), 7.0, dtype=torch.float32, device=gpu)
+    qwq4.gemv(dW, dS, dZ, x, N, K, M, y=y)
+    assert rel_err(host(y), oracle.q4_linear(W, S, Z, N, K, xf)) <= 1e-5  # fp32 sums of exact products

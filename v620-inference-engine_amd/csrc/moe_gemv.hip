@@ -118,8 +118,8 @@ __device__ __forceinline__ void moe_gate_up_gemv_block(
     auto chunk = [&](int m0) {
         const int mc = min(R, M - m0);
         // (stage_rows_issue asks for one row at a time, wave-uniform, when a
-        // row is whole waves of 16-byte pieces; else per lane)
-        const bool rows_uniform = (H / 8) % WAVE == 0;
+        // row has a wave of 16-byte pieces; else per lane)
+        const bool rows_uniform = H / 8 >= WAVE;
         stage_rows_issue(
             [&](int m) {
                 const int i = base + m0 + m;

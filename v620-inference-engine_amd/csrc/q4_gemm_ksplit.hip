@@ -43,6 +43,9 @@ bool launch_gemm_ksplit(const GemmArgs &a, const uint16_t *Xh, int lda, int cus,
     // against 171). Token rows within a tile are addressed by 32-bit offsets.
     const int64_t nb128 = (int64_t(a.N) + 255) / 256 * ((int64_t(a.T) + 127) / 128);
     if (nb128 >= 2 * int64_t(cus) || lda > (1 << 23)) return false;
+    // exactly one round of 256 x 128 tiles keeps every CU at its largest tile
+    // (2048 rows of K = 3712, 4050 tokens: 3% faster than the K-split tiles)
+    if ((int64_t(a.N) + 127) / 128 * ((int64_t(a.T) + 255) / 256) == cus) return false;
     int best = 0;
     float t = 0.f;
     for (int i = 0; i < int(sizeof SHAPES / sizeof SHAPES[0]); ++i) {

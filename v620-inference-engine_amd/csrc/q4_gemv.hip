@@ -9,7 +9,7 @@ void launch_gemv_fit_f16(const GemvArgs &a, hipStream_t s);
 bool gemv_fits(int M, int K) {
     const int MB = M <= 16 ? 1 : 2;
     int KS, SUB, NW;
-    dense_split(K / QGROUP, KS, SUB, NW);
+    dense_split(K / QGROUP, 1 << 28, M, KS, SUB, NW);  // (many subtiles: the largest blocks)
     return dense_lds_bytes(M, K, MB, KS * SUB, KS) <= 160 * 1024;
 }
 

@@ -15,15 +15,15 @@
 namespace qwq4 {
 
 // LDS row stride, in 16-byte pieces, of staged activation rows of K
-// elements: K / 8, plus one piece when K / 8 is a multiple of 64. A b128 read
-// pass serves 16 lanes that read 16 different rows at the same column; with a
-// row stride that is a multiple of 256 bytes they would all hit the same
-// banks (a 16-way conflict at 16 rows), the extra piece spreads them over 16
-// bank groups. Padded rows are staged row by row (each wave instruction's
-// 64 pieces stay inside one row).
+// elements: K / 8 made odd (rows of at least 64 pieces). A b128 read pass
+// serves 16 lanes that read 16 different rows at the same column; K is a
+// multiple of 128 or nearly so, so K / 8 pieces would put the rows 256 or 512
+// bytes apart modulo the banks (up to a 16-way conflict), the extra piece
+// spreads them over 16 bank groups. Padding only rows of whole waves of
+// pieces (K a multiple of 512) left the others in conflict: X_STRIDE_FIGURES.
 __host__ __device__ inline int x_row_stride(int K) {
     const int kc = K / 8;
-    return kc % 64 == 0 ? kc + 1 : kc;
+    return kc >= WAVE ? kc | 1 : kc;
 }
 
 // 16-byte pieces of M staged rows, rounded to whole waves.
@@ -33,18 +33,31 @@ __host__ __device__ inline int x_pieces(int M, int K) { return (M * x_row_stride
 // xl + m * x_row_stride(K), by direct global->LDS loads (no registers; 1 KB
 // per wave instruction). Issued before the weight loads; the barrier that
 // follows those waits for both, so activations (L2) and weights (HBM) are
-// requested before anything waits. With padded rows the row address is
-// wave-uniform (row(m) may then come from a scalar load, which does not wait
+// requested before anything waits. With rows of 64 pieces or more the row
+// address is wave-uniform (row(m) may then come from a scalar load, which does not wait
 // behind vector loads in flight).
+// (Rows of 64 pieces or more go in wave instructions of 64 pieces of one
+// row. Where a row is not whole instructions, its last one ends with the row,
+// over pieces that the one before has brought already.)
 template <class RowFn>
 __device__ __forceinline__ void stage_rows_issue(RowFn row, int M, int K, uint4 *xl) {
-    const int kc = K / 8, wave = threadIdx.x / WAVE, lane = threadIdx.x % WAVE, nw = blockDim.x / WAVE;
+    const int kc = K / 8, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE), lane = threadIdx.x % WAVE,
+              nw = blockDim.x / WAVE;
     if (kc % WAVE == 0) {
         const int st = kc + 1;
         for (int m = 0; m < M; ++m) {
             const uint16_t *r = row(m);
             for (int c = wave * WAVE; c < kc; c += nw * WAVE)
                 __builtin_amdgcn_global_load_lds(r + (c + lane) * 8, xl + m * st + c, 16, 0, 0);
+        }
+    } else if (kc > WAVE) {
+        const int st = x_row_stride(K);
+        for (int m = 0; m < M; ++m) {
+            const uint16_t *r = row(m);
+            for (int c0 = wave * WAVE; c0 < kc; c0 += nw * WAVE) {
+                const int c = min(c0, kc - WAVE);
+                __builtin_amdgcn_global_load_lds(r + (c + lane) * 8, xl + m * st + c, 16, 0, 0);
+            }
         }
     } else {
         const int total = M * kc;
@@ -65,9 +78,10 @@ __device__ __forceinline__ int opaque_lane() {
 }
 
 // A wave's whole K range of one subtile (groups g0 .. g0 + n - 1, n <= GW),
-// requested up front into registers. CH4: the range is whole 4-group chunks
-// (g0 and n multiples of 4), so each chunk's scales are one 8-byte load and
-// its zeros one 16-bit word; otherwise one scale and one zero load per group.
+// requested up front into registers. CH4: the range starts on a 4-group chunk
+// (g0 a multiple of 4; a last partial chunk is whole in the padded scale and
+// zero arrays), so each chunk's scales are one 8-byte load and its zeros one
+// 16-bit word; otherwise one scale and one zero load per group.
 // (A compile-time choice: a runtime branch between the two puts waits between
 // the loads.)
 template <int GW, bool HAS_Z, bool CH4 = false>
@@ -99,7 +113,7 @@ struct WaveRange {
             static_assert(GW % 4 == 0, "whole chunks");
 #pragma unroll
             for (int j = 0; j < GW / 4; ++j) {
-                const int gc = (g0 >> 2) + min(j, n / 4 - 1);
+                const int gc = (g0 >> 2) + min(j, (n + 3) / 4 - 1);
                 const uint2 s4 = *reinterpret_cast<const uint2 *>(t.s + gc * 64 + r * 4);
                 sv[2 * j] = s4.x;
                 sv[2 * j + 1] = s4.y;

@@ -82,6 +82,17 @@ __device__ __forceinline__ uint16_t swiglu_h(float g, float u, float gate) {
     return __builtin_bit_cast(uint16_t, f32_to_f16_satfinite(silu_ref(g) * u * gate));
 }
 
+// Row stride and pieces of the SwiGLU rows formed in LDS (padded only for K a
+// multiple of 512: the rows the entry point accepts are sized by it).
+__host__ __device__ inline int sg_row_stride(int K) {
+    const int kc = K / 8;
+    return kc % WAVE == 0 ? kc + 1 : kc;
+}
+__host__ __device__ inline int sg_pieces(int M, int K) { return (M * sg_row_stride(K) + WAVE - 1) / WAVE * WAVE; }
+__host__ __device__ inline size_t sg_lds_bytes(int M, int K, int MB, int KS) {
+    return size_t(sg_pieces(M, K)) * 16 + size_t(2) * red_slots(KS, KS) * MB * WAVE * 16;
+}
+
 struct SgPiece {
     float4 g0, g1, u0, u1;
     float gl;
@@ -104,7 +115,7 @@ __device__ __forceinline__ void sg_commit(const SgPiece &p, int n, int i, float 
     auto two = [&](float g0, float u0, float g1, float u1) {
         return uint32_t(swiglu_h(g0, u0, gate)) | (uint32_t(swiglu_h(g1, u1, gate)) << 16);
     };
-    xl[m * x_row_stride(n) + c] = make_uint4(two(p.g0.x, p.u0.x, p.g0.y, p.u0.y), two(p.g0.z, p.u0.z, p.g0.w, p.u0.w),
+    xl[m * sg_row_stride(n) + c] = make_uint4(two(p.g0.x, p.u0.x, p.g0.y, p.u0.y), two(p.g0.z, p.u0.z, p.g0.w, p.u0.w),
                                              two(p.g1.x, p.u1.x, p.g1.y, p.u1.y), two(p.g1.z, p.u1.z, p.g1.w, p.u1.w));
 }
 
@@ -116,10 +127,10 @@ __device__ __forceinline__ void w16_swiglu_block(const uint16_t *W, const float 
     const int tid = threadIdx.x, kp = __builtin_amdgcn_readfirstlane(tid / WAVE), lane = tid % WAVE, q = lane / 16,
               n = lane % 16;
     const int steps = K / 32, spw = (steps + KS - 1) / KS, s0 = kp * spw, ns = min(spw, steps - s0);
-    const int kc = x_row_stride(K), P = M * (K / 8), nt = blockDim.x;
+    const int kc = sg_row_stride(K), P = M * (K / 8), nt = blockDim.x;
     const float rkn = __builtin_amdgcn_rcpf(float(K / 8));
     uint4 *xl = reinterpret_cast<uint4 *>(smem);
-    float *red = reinterpret_cast<float *>(xl + x_pieces(M, K));
+    float *red = reinterpret_cast<float *>(xl + sg_pieces(M, K));
     SgPiece p0, p1, p2, p3;  // named, not an array (see XRegs)
     if constexpr (XPT >= 1) sg_load(v, ldv, K, min(tid, P - 1), rkn, p0);
     if constexpr (XPT >= 2) sg_load(v, ldv, K, min(tid + nt, P - 1), rkn, p1);

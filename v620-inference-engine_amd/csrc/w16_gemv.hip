@@ -178,7 +178,7 @@ __global__ __launch_bounds__(W16_MAX_KS *WAVE) void w16_swiglu_kernel(const uint
 template <int MB, int MR>
 static void launch_w16_swiglu_t(const W16SwigluArgs &a, hipStream_t s) {
     const int KS = w16_ks(a.n, a.N), threads = KS * WAVE;
-    const size_t lds = dense_lds_bytes(a.M, a.n, MB, KS, KS);
+    const size_t lds = sg_lds_bytes(a.M, a.n, MB, KS);
     const int xpt = (a.M * (a.n / 8) + threads - 1) / threads;
     const unsigned blocks = unsigned((a.N + 15) / 16);
     auto go = [&](auto kern) {
@@ -197,7 +197,9 @@ static void launch_w16_swiglu_t(const W16SwigluArgs &a, hipStream_t s) {
     else pick(std::integral_constant<int, 16>());
 }
 
-bool w16_swiglu_fits(int M, int n, int N) { return w16_fits(M, n, N); }
+bool w16_swiglu_fits(int M, int n, int N) {
+    return sg_lds_bytes(M, n, M > 16 ? 2 : 1, w16_ks(n, N)) <= 160 * 1024;
+}
 
 void launch_w16_swiglu(const W16SwigluArgs &a, hipStream_t s) {
     if (a.M > 16) launch_w16_swiglu_t<2, 4>(a, s);

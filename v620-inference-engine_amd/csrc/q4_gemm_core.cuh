@@ -88,6 +88,14 @@ struct BRow {
     }
 };
 
+// both halves' rows of a value each lane holds for its own row (rows 0-31 in
+// lanes 0-31, 32-63 in lanes 32-63): a = row lane % 32, b = row 32 + lane % 32
+__device__ __forceinline__ void split_halves(uint32_t v, uint32_t &a, uint32_t &b) {
+    const auto r = __builtin_amdgcn_permlane32_swap(v, v, false, false);
+    a = r[0];
+    b = r[1];
+}
+
 constexpr int G_ROLE = G_WAVES / 2;  // waves per loading role
 
 // The four stage buffers (A and weights, two stages each), at file scope so
@@ -280,16 +288,19 @@ __device__ __forceinline__ void gemm_tile(const uint16_t *const *ap, const BRow 
 // row, 64 j + 8 w + lane / 8; rows past BM none). Four-wave blocks of 256
 // weight rows (two blocks per CU) measured slower (down GEMM 835 against
 // 661 us).
+// Scales and zeros are loaded once per 128-K group, of the lane's own row
+// (bs), and crossed between the wave's halves in a register swap, instead of
+// both groups' with every stage: two to four loads fewer per 128 K and lane,
+// 250 tokens over 256 experts 565 -> 554 us, 4096 tokens 1645 -> 1639.
 // (USE: a tag per call site; the host pass rejects one specialization
 // called from two kernels' device code)
 template <int BM, bool HAS_Z, int USE>
 __device__ __forceinline__ void gemm_tile_rd2(const uint16_t *const (&arow)[(BM + 63) / 64], const BRow &b0,
-                                              const BRow &b1, int K, f32x16 (&acc)[BM / 32][2]) {
+                                              const BRow &b1, const BRow &bs, int K, f32x16 (&acc)[BM / 32][2]) {
     static_assert(BM % 32 == 0 && BM <= 160, "tiles of 32 to 160 rows");
     constexpr int NI = BM / 32, NA = (BM + 63) / 64;
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid / WAVE), lane = tid % WAVE;
     const int l32 = lane % 32, lh = lane / 32, nk = K / GB_K;
-    constexpr int NLD = HAS_Z ? 6 : 4;  // weight-side loads per stage and lane
     auto bufA = [&](int i) { return i ? lds_a1 : lds_a0; };
     auto issue_a = [&](int ks, unsigned char *dst) {
 #pragma unroll
@@ -299,31 +310,35 @@ __device__ __forceinline__ void gemm_tile_rd2(const uint16_t *const (&arow)[(BM 
                 __builtin_amdgcn_global_load_lds(arow[j] + ks * GB_K + c * 8, dst + rb * 128, 16, 0, 0);
         }
     };
+    // raw weights of a stage; with an even stage also its group's scale and
+    // zero word, of the lane's own row (bs: row 64 w + lane)
     struct WR {
         uint4 w0, w1;
-        uint16_t s0, s1;
-        uint32_t z0, z1;
     };
-    auto issue_w = [&](int ks, WR &r) {
-        ks = min(ks, nk - 1);  // past the end: a valid (unused) load
-        const int g = ks / 2, e = g * 64 + ((ks % 2) * 2 + lh) * 16, so = (g >> 2) * 64 + (g & 3);
+    uint16_t rs = 0;
+    uint32_t rz = 0;
+    constexpr int NLE = 3 + HAS_Z, NLO = 2;  // weight-side loads of an even and an odd stage
+    auto issue_w = [&](int ks, WR &r, bool even) {
+        ks = min(ks, nk - 2 + !even);  // past the end: a valid (unused) load
+        const int g = ks / 2, e = g * 64 + ((ks % 2) * 2 + lh) * 16;
         r.w0 = b0.w[e];
         r.w1 = b1.w[e];
-        r.s0 = b0.s[so];
-        r.s1 = b1.s[so];
-        if constexpr (HAS_Z) {
-            r.z0 = b0.z[(g >> 2) * 8];
-            r.z1 = b1.z[(g >> 2) * 8];
+        if (even) {
+            rs = bs.s[(g >> 2) * 64 + (g & 3)];
+            if constexpr (HAS_Z) rz = bs.z[(g >> 2) * 8];
         }
     };
-    auto compute = [&](const unsigned char *a, const WR &r, int ks) {
-        uint32_t s0 = r.s0, s1 = r.s1, z0 = HAS_Z ? r.z0 : 0u, z1 = HAS_Z ? r.z1 : 0u;
-        asm volatile("" : "+v"(s0), "+v"(s1), "+v"(z0), "+v"(z1));  // taken here, not at their loads (see commit_b)
-        const int g = ks / 2;
-        const h2 zb0 = zero_bias(HAS_Z ? (z0 >> (b0.zs + 4 * (g & 3))) & 0xfu : 8u);
-        const h2 zb1 = zero_bias(HAS_Z ? (z1 >> (b1.zs + 4 * (g & 3))) & 0xfu : 8u);
-        const _Float16 c0 = __builtin_bit_cast(_Float16, uint16_t(s0)), c1 = __builtin_bit_cast(_Float16, uint16_t(s1));
-        const h2 sa = {c0, c0}, sb = {c1, c1};
+    // the group's packed scales and 1024 + z of both row groups
+    uint32_t sv0, sv1, zv0 = 0x64086408u, zv1 = 0x64086408u;
+    auto open_group = [&](int ks) {
+        uint32_t s = rs, z = rz;
+        asm volatile("" : "+v"(s), "+v"(z));  // taken here, not at their loads (see commit_b)
+        split_halves(s * 0x10001u, sv0, sv1);
+        if constexpr (HAS_Z) split_halves(((z >> (bs.zs + 4 * ((ks / 2) & 3))) & 0xfu) * 0x10001u | 0x64006400u, zv0, zv1);
+    };
+    auto compute = [&](const unsigned char *a, const WR &r) {
+        const h2 zb0 = __builtin_bit_cast(h2, zv0), zb1 = __builtin_bit_cast(h2, zv1);
+        const h2 sa = __builtin_bit_cast(h2, sv0), sb = __builtin_bit_cast(h2, sv1);
         const uint32_t wa[4] = {r.w0.x, r.w0.y, r.w0.z, r.w0.w}, wb[4] = {r.w1.x, r.w1.y, r.w1.z, r.w1.w};
         uint4 af[NI], an[NI];
         auto rd = [&](int kk, uint4 (&f)[NI]) {
@@ -346,20 +361,22 @@ __device__ __forceinline__ void gemm_tile_rd2(const uint16_t *const (&arow)[(BM 
     };
     WR w0, w1;
     issue_a(0, bufA(0));
-    issue_w(0, w0);
-    issue_w(1, w1);
-    wait_vm_below<NLD>();  // A(0) and W(0) here; W(1) stays in flight
+    issue_w(0, w0, true);
+    issue_w(1, w1, false);
+    wait_vm_below<NLO>();  // A(0) and W(0) here; W(1) stays in flight
     __builtin_amdgcn_s_barrier();
-    auto stage = [&](int ks, int p, WR &cur) {
-        issue_a(min(ks + 1, nk - 1), bufA(p ^ 1));
-        compute(bufA(p), cur, ks);
-        issue_w(ks + 2, cur);
-        wait_vm_below<NLD>();  // everything but W(ks + 2): A(ks + 1) and W(ks + 1) arrived
-        __builtin_amdgcn_s_barrier();
-    };
     for (int ks = 0; ks < nk; ks += 2) {  // nk is even (K is a multiple of 128)
-        stage(ks, 0, w0);
-        stage(ks + 1, 1, w1);
+        issue_a(min(ks + 1, nk - 1), bufA(1));
+        open_group(ks);
+        compute(bufA(0), w0);
+        issue_w(ks + 2, w0, true);
+        wait_vm_below<NLE>();  // everything but W(ks + 2): A(ks + 1) and W(ks + 1) arrived
+        __builtin_amdgcn_s_barrier();
+        issue_a(min(ks + 2, nk - 1), bufA(0));
+        compute(bufA(1), w1);
+        issue_w(ks + 3, w1, false);
+        wait_vm_below<NLO>();
+        __builtin_amdgcn_s_barrier();
     }
 }
 

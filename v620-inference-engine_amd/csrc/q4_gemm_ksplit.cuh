@@ -35,14 +35,6 @@ struct KSplit {
     static_assert(PER >= 1 && PER * NST >= 8, "the partial sums fit the stage buffers");
 };
 
-// both halves' rows of a value each lane holds for its own row (rows 0-31 in
-// lanes 0-31, 32-63 in lanes 32-63): a = row lane % 32, b = row 32 + lane % 32
-__device__ __forceinline__ void split_halves(uint32_t v, uint32_t &a, uint32_t &b) {
-    const auto r = __builtin_amdgcn_permlane32_swap(v, v, false, false);
-    a = r[0];
-    b = r[1];
-}
-
 // one output element as stored (yt: 0 fp32, 1 bf16, 2 fp16 saturated)
 __device__ __forceinline__ uint32_t cvt_y16(float v, int yt) {
     return yt == 1 ? f32_to_bf16_rne(v) : __builtin_bit_cast(uint16_t, f32_to_f16_satfinite(v));

@@ -200,3 +200,52 @@ def test_gemv_ragged_k(gpu, oracle, N, K, M, f16):
     y = torch.full((M, N), 7.0, dtype=torch.float32, device=gpu)
     qwq4.gemv(dW, dS, dZ, x, N, K, M, y=y)
     assert rel_err(host(y), oracle.q4_linear(W, S, Z, N, K, xf)) <= 1e-5  # fp32 sums of exact products
+
+
+# Rows streamed in K groups (batches of 9 to 32 whose rows do not fit LDS):
+# one and two 16-row blocks, a K split with unequal parts (43 groups) and
+# equal ones, 64- and 128- or 256-row blocks (N above 64 Ki rows), weight rows off
+# every block size.
+@pytest.mark.parametrize("N,K,M", [(1040, 6144, 12), (16, 11008, 16), (4112, 5504, 17), (528, 4096, 32), (3076 // 16 * 16, 3712, 25),
+                                   (65584, 6144, 9), (32848, 4096, 21)])
+@pytest.mark.parametrize("f16,zeros", [(False, True), (True, True), (False, False), (True, False)])
+def test_gemv_wide(gpu, oracle, N, K, M, f16, zeros):
+    import torch
+    print(f"gemv wide N={N} K={K} M={M} f16={f16} zeros={zeros}", flush=True)
+    g = torch.Generator(device=gpu)
+    g.manual_seed(N + K)
+    W = torch.randint(-2**31, 2**31, (N, K // 8), generator=g, device=gpu, dtype=torch.int32)
+    S = (torch.randn((N, K // 128), generator=g, device=gpu) * 0.02).abs().to(torch.float16)
+    Z = torch.randint(-2**31, 2**31, (N, (K // 128 + 7) // 8), generator=g, device=gpu, dtype=torch.int32) if zeros else None
+    d = qwq4.tile(W, S, Z, N, K)
+    x = torch.full((M, K + 64), float("nan"), device=gpu).to(torch.float16 if f16 else torch.bfloat16)
+    x[:, :K] = torch.randn((M, K), generator=g, device=gpu).to(x.dtype)
+    y = torch.full((M, N + 3), 7.0, dtype=torch.float32, device=gpu)
+    qwq4.gemv(*d, x, N, K, M, y=y)
+    assert bool((y[:, N:] == 7.0).all())
+    rows = np.unique(np.r_[0, N - 1, np.random.default_rng(N).choice(N, min(N, 512), replace=False)])
+    np_ = lambda t, v: None if t is None else host(t[torch.from_numpy(rows).to(gpu)]).view(v)
+    ref = oracle.q4_linear_f64(np_(W, np.uint32), np_(S, np.uint16), np_(Z, np.uint32), len(rows), K, host(x[:, :K].float().contiguous()))
+    assert rel_err(host(y)[:, rows], ref) <= 1e-5  # fp32 sums of exact products
+    acc = y.clone()
+    qwq4.gemv(*d, x, N, K, M, y=acc, accumulate=True)
+    assert torch.equal(acc[:, :N], 2 * y[:, :N])
+    yb = torch.zeros((M, N), dtype=torch.bfloat16, device=gpu)
+    qwq4.gemv(*d, x, N, K, M, y=yb, y_bf16=True)
+    assert torch.equal(yb, y[:, :N].to(torch.bfloat16))
+
+
+def test_gemv_wide_row_slices(gpu):
+    """Rows grouped over activation slices: each equals the ungrouped product
+    with its slice, bit for bit, whichever block sizes its slice alone would get."""
+    import torch
+    N, K, M, rpg = 36864, 4096, 20, 3076
+    print("gemv wide row slices", flush=True)
+    W, S, Z = synth.q4_weights(93, "wrs", N, K)
+    d = qwq4.tile(to_dev(W, gpu), to_dev(S, gpu), to_dev(Z, gpu), N, K)
+    ns = -(-N // rpg)
+    x = torch.randn((M, ns * K), device=gpu).to(torch.bfloat16)
+    y = qwq4.gemv(*d, x, N, K, M, rpg=rpg)
+    for sl in (0, 5, ns - 1):
+        whole = qwq4.gemv(*d, x[:, sl * K:(sl + 1) * K], N, K, M)
+        assert torch.equal(y[:, sl * rpg:(sl + 1) * rpg], whole[:, sl * rpg:(sl + 1) * rpg])

@@ -20,7 +20,7 @@
 // rounding); products and sums run on the fp16 MFMA with fp32 accumulation.
 #pragma once
 
-#include "q4_common.cuh"
+#include "q4_lanes.cuh"
 
 namespace qwq4 {
 
@@ -39,8 +39,6 @@ constexpr size_t GEMM_LDS = 4 * size_t(TILE_BYTES);  // the stage buffers (stati
 // to the reads.
 __device__ __forceinline__ int swz_x(int r) { return (r & 7) ^ ((r >> 3) & 1); }
 __device__ __forceinline__ int swz(int r, int c) { return r * 128 + ((c ^ swz_x(r)) << 4); }
-
-typedef _Float16 h2 __attribute__((ext_vector_type(2)));
 
 // 8 packed nibbles (tiled word) -> 8 fp16 weights (q - z) * s: the nibbles
 // become fp16 1024 + q (unpack8 with no byte offset), 1024 + z is subtracted
@@ -87,14 +85,6 @@ struct BRow {
         zs = (n & 1) * 16;
     }
 };
-
-// both halves' rows of a value each lane holds for its own row (rows 0-31 in
-// lanes 0-31, 32-63 in lanes 32-63): a = row lane % 32, b = row 32 + lane % 32
-__device__ __forceinline__ void split_halves(uint32_t v, uint32_t &a, uint32_t &b) {
-    const auto r = __builtin_amdgcn_permlane32_swap(v, v, false, false);
-    a = r[0];
-    b = r[1];
-}
 
 constexpr int G_ROLE = G_WAVES / 2;  // waves per loading role
 

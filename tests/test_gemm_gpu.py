@@ -286,7 +286,7 @@ def test_gemm_ksplit_nonfinite(gpu, oracle):
 # the block sizes: experts of 1, 16, 17, 32, 33 and over 160 tokens beside
 # empty ones; F and H off the 256- and 512-row blocks, an odd number of K groups.
 @pytest.mark.parametrize("yp16", [False, True])
-@pytest.mark.parametrize("E,H,F,zeros", [(96, 384, 640, True), (64, 1152, 128, False), (128, 512, 384, True)])
+@pytest.mark.parametrize("E,H,F,zeros", [(96, 384, 640, True), (64, 640, 128, False), (128, 512, 384, True)])
 def test_grouped_light_loads(gpu, oracle, E, H, F, zeros, yp16):
     print(f"grouped light E={E} H={H} F={F} zeros={zeros} yp16={yp16}", flush=True)
     want = {3: 1, 5: 16, 9: 17, 20: 32, 33: 33, 50: 170, E - 1: 5}
@@ -301,7 +301,6 @@ def test_grouped_light_loads(gpu, oracle, E, H, F, zeros, yp16):
     out, h_ref, yp_ref = oracle.moe(xf, l, k, *ex, want_parts=True)
     from test_moe_gpu import _experts_dev
     (dg, du, dd), E, F = _experts_dev(gpu, ex)
-    assert T * k <= 24 * E
     r = qwq4.moe_route(to_dev(l, gpu), k, tile_m=qwq4.moe_grouped_tile_m())
     h, yp = qwq4.moe_experts_grouped(dg, du, dd, r, to_dev(xb, gpu), E, F, yp_f16=yp16)
     assert rel_err(host(h).astype(np.float32), h_ref) <= TOL

@@ -207,3 +207,27 @@ def test_moe_decode_random_small_batches(gpu, T, E, H, F, k):
     o2 = qwq4.moe_combine(yp, r, H, shared=to_dev(sh, gpu), out_bf16=False)
     assert np.array_equal(host(yp), host(buf.yp))
     assert np.array_equal(host(out).view(np.uint32), host(o2).view(np.uint32))
+
+
+# Down projections of 6 to 11 K groups (parts of 3 + 3, 4 + 3, 5 + 4, 5 + 5 and
+# 6 + 5 groups) and of one: the block equal, bit for bit, to its separate calls
+# and within the tolerance of the oracle.
+@pytest.mark.parametrize("F", [128, 768, 896, 1152, 1280, 1408])
+@pytest.mark.parametrize("T,zeros", [(1, True), (2, False), (3, True), (9, False)])
+def test_moe_decode_down_parts(gpu, oracle, F, T, zeros):
+    import torch
+    E, H, k = 16, 512, 4
+    print(f"moe decode parts F={F} T={T}", flush=True)
+    ex = synth.experts(77, E, H, F, zeros=zeros)
+    from test_moe_gpu import _experts_dev
+    (dg, du, dd), E, F = _experts_dev(gpu, ex)
+    xb, xf = synth.acts(77, f"dp{T}", T, H)
+    rw = np.random.default_rng(F + T).standard_normal((E, H)).astype(np.float32) * 0.05
+    x = to_dev(xb, gpu)
+    out, buf = qwq4.moe_decode(torch.from_numpy(rw).to(gpu), x, k, dg, du, dd, E, F, out_bf16=False)
+    r = qwq4.moe_route(buf.logits, k)
+    h, yp = qwq4.moe_experts_gemv(dg, du, dd, r, x, E, F)
+    sep = qwq4.moe_combine(yp, r, H, out_bf16=False)
+    assert torch.equal(r.top_e, buf.top_e) and torch.equal(h, buf.h) and torch.equal(yp, buf.yp)
+    assert torch.equal(sep, out)
+    assert rel_err(host(out), oracle.moe(xf, host(buf.logits), k, *ex)) <= TOL

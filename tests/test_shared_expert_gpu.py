@@ -367,3 +367,11 @@ def test_moe_decode_with_shared_random_shapes(gpu, T, E, H, F, k, SF, f16, zeros
     assert np.array_equal(host(sv).view(np.uint32), host(v).view(np.uint32))
     assert np.array_equal(host(so).view(np.uint32), host(sh).view(np.uint32))
     assert np.array_equal(host(out).view(np.uint32), host(o2).view(np.uint32))
+
+
+# Shared experts that are not whole steps of the GEMV's 8 waves (Fs / 32 = 9, 20, 36,
+# 44), merged at batch 1, 2-4, 5-8 and above, and one below the merged launches.
+@pytest.mark.parametrize("SF", [128, 288, 640, 1152, 1408])
+@pytest.mark.parametrize("T,f16,zeros", [(1, True, False), (3, False, True), (7, True, True), (12, False, False)])
+def test_moe_decode_with_shared_ragged_fs(gpu, T, SF, f16, zeros):
+    test_moe_decode_with_shared_random_shapes(gpu, T, 32, 2048, 384, 4, SF, f16, zeros)

@@ -403,11 +403,11 @@ __global__ __launch_bounds__(512) void moe_down_gemv_kernel(const uint32_t *dw, 
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid / WAVE), lane = tid % WAVE, q = lane / 16,
               n = lane % 16;
     const int sl = wave / KS, kp = wave % KS;
-    const int G = F / QGROUP, gpk = G / KS, hsub = H / 16, kc = x_row_stride(F);
+    const int G = F / QGROUP, gpk = (G + KS - 1) / KS, ng = min(gpk, G - kp * gpk), hsub = H / 16, kc = x_row_stride(F);
     const int lsub = blockIdx.x * SUB + sl;
     const Q4Tile t(dw, ds, dz, int64_t(e) * hsub + min(lsub, hsub - 1), G);
     WaveRange<GW, HAS_Z, CH4> wr;
-    wr.fetch(t, kp * gpk, gpk, opaque_lane());
+    wr.fetch(t, kp * gpk, ng, opaque_lane());
     const int base = ld_uniform(offsets, e), M = ld_uniform(offsets, e + 1) - base;
     uint4 *xl = reinterpret_cast<uint4 *>(smem);
     f32x4 *red = reinterpret_cast<f32x4 *>(xl + x_pieces(R, F));
@@ -450,7 +450,7 @@ __global__ __launch_bounds__(512) void moe_down_gemv_kernel(const uint32_t *dw, 
     chunk(0);
     if constexpr (MULTI) {
         for (int m0 = R; m0 < M; m0 += R) {
-            wr.fetch(t, kp * gpk, gpk, opaque_lane());
+            wr.fetch(t, kp * gpk, ng, opaque_lane());
             lds_barrier();
             chunk(m0);
         }
@@ -526,10 +526,10 @@ __global__ __launch_bounds__(1024) void moe_down_t1_kernel(const uint32_t *dw, c
     const int rows = min(na, topk);
     const bool live = y < rows;  // wave-uniform
     const int e = live ? min(max(ea, 0), E - 1) : 0;
-    const int G = F / QGROUP, gpk = G / 2, hsub = H / 16, kc = x_row_stride(F);
+    const int G = F / QGROUP, gpk = (G + 1) / 2, ng = min(gpk, G - kp * gpk), hsub = H / 16, kc = x_row_stride(F);
     const Q4Tile t(dw, ds, dz, int64_t(e) * hsub + blockIdx.x, G);
     WaveRange<GW, HAS_Z, CH4> wr;
-    wr.fetch(t, kp * gpk, gpk, opaque_lane());
+    wr.fetch(t, kp * gpk, ng, opaque_lane());
     // the combine's inputs, requested now so that their latency is hidden:
     // the selections' slots and weights (block-uniform, scalar loads) and
     // the shared row's values (wave 0)
@@ -577,12 +577,13 @@ static int pick_ks(int G, int kmax) {
     return ks;
 }
 
-// Down projection: a split of 2 where a wave's range stays within 16
-// groups (fewer, larger blocks: each has more weight bytes in flight for its
-// fixed costs), else up to 8.
+// Down projection: a split of 2 where a wave's range stays within 16 groups
+// (fewer, larger blocks: each has more weight bytes in flight for its fixed
+// costs), else up to 8; the last part takes what is left. (Equal parts left odd
+// group counts unsplit, 128 rows per block: DOWN_ODD_F.)
 static int down_ks(int G) {
-    int ks = pick_ks(G, 2);
-    while (G / ks > 16 && ks < 8 && G % (ks * 2) == 0) ks *= 2;
+    int ks = G > 1 ? 2 : 1;
+    while ((G + ks - 1) / ks > 16 && ks < 8) ks *= 2;
     return ks;
 }
 
@@ -648,7 +649,7 @@ bool launch_gate_up_routed_shdown(const MoeGemvArgs &a, const ShExpertArgs &sh, 
         using XT = decltype(xt);
         constexpr int GW = decltype(gw)::value, PER = decltype(pr)::value;
         constexpr bool HZ = decltype(hz)::value;
-        if (sh.Fs / 32 / W16_MAX_KS <= 8) go(gate_up_routed_shdown_kernel<XT, GW, HZ, PER, 8>);
+        if ((sh.Fs / 32 + W16_MAX_KS - 1) / W16_MAX_KS <= 8) go(gate_up_routed_shdown_kernel<XT, GW, HZ, PER, 8>);
         else go(gate_up_routed_shdown_kernel<XT, GW, HZ, PER, 16>);
     };
     auto by_per = [&](auto xt, auto gw, auto hz) {
@@ -698,7 +699,7 @@ bool launch_gate_up_shdown(const MoeGemvArgs &a, const ShExpertArgs &sh, const u
     // the gate/up shapes of launch_gw with the K split in 4: 4 or 8 groups per
     // wave, whole 4-group chunks (H 2048 and 4096)
     if (a.route_logits || a.T < 5 || a.T > 32 || pick_ks(G, 4) != 4 || (G / 4 != 4 && G / 4 != 8) ||
-        sh.Fs % 256 != 0 || (a.gz != nullptr) != (a.uz != nullptr) || !w16_fits(a.T, sh.Fs, a.H))
+        sh.Fs % 32 != 0 || sh.Fs < 256 || (a.gz != nullptr) != (a.uz != nullptr) || !w16_fits(a.T, sh.Fs, a.H))
         return false;
     // the gate/up launch's shape (launch_one, launch_gate_up): rows per chunk
     // as many as keep the staged activations within 32 KB
@@ -840,9 +841,21 @@ static void launch_kind(const MoeGemvArgs &a, int max_active, int R, hipStream_t
 
 template <bool DOWN, int KS, bool HAS_Z>
 static void launch_gw(const MoeGemvArgs &a, int max_active, int R, int gpk, hipStream_t s) {
+    // (a range shorter than GW requests its last group again: the down parts
+    // of F = 768 and 1152, 1280 have their own sizes)
+    if constexpr (DOWN) {
+        if (gpk == 3) {
+            launch_kind<DOWN, KS, 3, HAS_Z, false>(a, max_active, R, s);
+            return;
+        }
+        if (gpk == 5) {
+            launch_kind<DOWN, KS, 5, HAS_Z, false>(a, max_active, R, s);
+            return;
+        }
+    }
     if (gpk == 4) launch_kind<DOWN, KS, 4, HAS_Z, true>(a, max_active, R, s);
     else if (gpk < 4) launch_kind<DOWN, KS, 4, HAS_Z, false>(a, max_active, R, s);
-    else if (gpk == 6) launch_kind<DOWN, KS, 6, HAS_Z, false>(a, max_active, R, s);  // down at F = 1536
+    else if (gpk == 6) launch_kind<DOWN, KS, 6, HAS_Z, false>(a, max_active, R, s);  // down at F = 1536 (1408: 6 + 5)
     else if (gpk == 8) launch_kind<DOWN, KS, 8, HAS_Z, true>(a, max_active, R, s);
     else if (gpk < 8) launch_kind<DOWN, KS, 8, HAS_Z, false>(a, max_active, R, s);
     else if (gpk % 4 == 0) launch_kind<DOWN, KS, 16, HAS_Z, true>(a, max_active, R, s);
@@ -853,7 +866,7 @@ template <bool DOWN, bool HAS_Z>
 static void launch_one(const MoeGemvArgs &a, int max_active, hipStream_t s) {
     const int K = DOWN ? a.F : a.H, G = K / QGROUP;
     const int ks = DOWN ? down_ks(G) : pick_ks(G, 4);
-    const int gpk = G / ks;
+    const int gpk = (G + ks - 1) / ks;
     // rows per block: a decode batch's tokens of one expert, as many as keep
     // the staged activations within 32 KB (two blocks per CU)
     int R = a.T < 16 ? a.T : 16;
@@ -874,8 +887,14 @@ int moe_down_row_blocks(int H, int F) {
 }
 
 bool moe_gemv_supported(int H, int F) {
-    // each wave holds at most 16 groups of its K range
-    return H / QGROUP / pick_ks(H / QGROUP, 4) <= 16 && F / QGROUP / down_ks(F / QGROUP) <= 16;
+    // each wave holds at most 16 groups of its K range, in equal parts (the
+    // sizes the entry points take; the down projection splits unequally too)
+    auto parts = [](int G) {
+        int ks = pick_ks(G, 2);
+        while (G / ks > 16 && ks < 8 && G % (ks * 2) == 0) ks *= 2;
+        return ks;
+    };
+    return H / QGROUP / pick_ks(H / QGROUP, 4) <= 16 && F / QGROUP / parts(F / QGROUP) <= 16;
 }
 
 void launch_moe_down(const MoeGemvArgs &a, hipStream_t s) {

@@ -376,12 +376,19 @@ __global__ __launch_bounds__(G_THREADS, 4) void moe_down_light_kernel(
     else down_light<2, HAS_Z, YP16>(dw, ds, dz, e, base + c0, min(32, M - c0), h, H, F, yp);
 }
 
-// Few tokens per expert on average: the light kernels. Same box, both expert
-// GEMMs, tiles of up to 160 slots against these (256 experts of 4096 / 1536,
-// top 8, uneven loads): 80 tokens (2.5 per expert) 446 -> 351 us, 250 (7.8)
-// 533 -> 454, 600 (19) 655 -> 623, 900 (28) 725 -> 761; 128 experts of 3072 /
-// 896 with zeros, top 6: 500 tokens (23) 207 -> 197, 700 (33) 227 -> 234.
-static bool light_load(int T, int topk, int E) { return int64_t(T) * topk <= int64_t(24) * E; }
+// Few tokens per expert on average: the light kernels, up to 20 where their
+// gate/up blocks fill the chip, fewer where they leave CUs with one block or
+// none (its groups then wait for their loads one by one; the longer K, the
+// more). Same box, both expert GEMMs, tiles of up to 160 slots against these:
+// 256 experts of 4096 / 1536, top 8, uneven loads, 2.5 tokens per expert
+// 446 -> 351 us, 7.8 533 -> 454, 19 655 -> 623, 28 725 -> 761; 128 experts of
+// 4096 / 1024 with zeros, 8 per expert 212 -> 191, 14 235 -> 241; 64 experts of
+// 4096 / 768, 4 per expert 84 -> 75, 8 97 -> 113; 64 of 2048 / 1408, 17 per
+// expert 98 -> 90.
+static bool light_load(int T, int topk, int E, int H, int F) {
+    const int64_t fill = int64_t((F + 255) / 256) * E * 4096 / H;  // gate/up blocks, at 4096 K
+    return int64_t(T) * topk <= (fill >= 640 ? 20 : fill >= 320 ? 12 : 6) * int64_t(E);
+}
 
 void launch_moe_grouped(const MoeGroupedArgs &a, hipStream_t s) {
     // bf16 rows through the fp16 pre-pass into the workspace; fp16 rows as they are
@@ -394,7 +401,7 @@ void launch_moe_grouped(const MoeGroupedArgs &a, hipStream_t s) {
     const int max_tiles = a.T * a.topk / -GROUPED_TILE_M + a.E;
     const dim3 g1(unsigned((a.F + 255) / 256), unsigned(max_tiles)), g2(unsigned((a.H + 511) / 512), unsigned(max_tiles));
     const GateUpTile gu{a.gw, a.uw, a.gs, a.gz, a.us, a.uz, a.pair_tok, xh, a.H, a.F, a.h};
-    if (light_load(a.T, a.topk, a.E)) {
+    if (light_load(a.T, a.topk, a.E, a.H, a.F)) {
         const dim3 l1(g1.x, g1.y, 5), l2(g2.x, g2.y, 5);
         auto gate_up = a.gz ? moe_gate_up_light_kernel<true> : moe_gate_up_light_kernel<false>;
         gate_up<<<l1, G_THREADS, 0, s>>>(gu, a.offsets, a.tile_e, a.tile_m0, a.n_tiles);

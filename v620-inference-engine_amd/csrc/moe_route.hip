@@ -582,7 +582,7 @@ __global__ __launch_bounds__(8 * WAVE) void router_logits_shgu_kernel(RouteArgs 
 }
 
 bool shared_logits_ok(int T, int H, int Fs) {
-    return T >= 1 && T <= 8 && H % 256 == 0 && H <= 8192 && Fs % 256 == 0 && Fs <= 4096;
+    return T >= 1 && T <= 8 && H % 256 == 0 && H <= 8192 && Fs % 32 == 0 && Fs >= 256 && Fs <= 4096;
 }
 
 void launch_router_logits_shgu(const RouterArgs &r, int T, int E, const ShExpertArgs &sh, hipStream_t s) {
@@ -872,7 +872,7 @@ __global__ __launch_bounds__(8 * WAVE) void route_shdown_kernel(RouteArgs a, ShE
 
 bool launch_route_shdown(const RouteArgs &a, const ShExpertArgs &sh, int H, hipStream_t s) {
     const int T = a.T, Fs = sh.Fs;
-    if (T < 2 || T > 4 || a.E > 8 * WAVE || a.tile_m != 0 || Fs % 256 != 0 || !w16_swiglu_fits(T, Fs, H)) return false;
+    if (T < 2 || T > 4 || a.E > 8 * WAVE || a.tile_m != 0 || Fs % 32 != 0 || Fs < 256 || !w16_swiglu_fits(T, Fs, H)) return false;
     const size_t lds = dense_lds_bytes(T, Fs, 1, W16_MAX_KS, W16_MAX_KS);
     if (lds + ROUTE_STATIC_LDS > 160 * 1024) return false;
     const unsigned grid = unsigned(1 + (H + 15) / 16);

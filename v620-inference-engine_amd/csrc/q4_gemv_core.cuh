@@ -40,9 +40,8 @@ __host__ __device__ inline int x_pieces(int M, int K) { return (M * x_row_stride
 // row. Where a row is not whole instructions, its last one ends with the row,
 // over pieces that the one before has brought already.)
 template <class RowFn>
-__device__ __forceinline__ void stage_rows_issue(RowFn row, int M, int K, uint4 *xl) {
-    const int kc = K / 8, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE), lane = threadIdx.x % WAVE,
-              nw = blockDim.x / WAVE;
+__device__ __forceinline__ void stage_rows_issue(RowFn row, int M, int K, uint4 *xl, int nw) {
+    const int kc = K / 8, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE), lane = threadIdx.x % WAVE;
     if (kc % WAVE == 0) {
         const int st = kc + 1;
         for (int m = 0; m < M; ++m) {
@@ -66,6 +65,11 @@ __device__ __forceinline__ void stage_rows_issue(RowFn row, int M, int K, uint4 
             __builtin_amdgcn_global_load_lds(row(m) + c * 8, xl + base, 16, 0, 0);
         }
     }
+}
+
+template <class RowFn>
+__device__ __forceinline__ void stage_rows_issue(RowFn row, int M, int K, uint4 *xl) {
+    stage_rows_issue(row, M, K, xl, int(blockDim.x) / WAVE);
 }
 
 // The lane index, as a value the compiler cannot see through: per-lane

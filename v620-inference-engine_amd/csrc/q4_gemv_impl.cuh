@@ -44,7 +44,7 @@ template <typename XT, int NW, int MB, bool HAS_Z, bool PF, bool KSNW, int XPT, 
 // Argument order: what the weight and activation requests need first (the
 // first 14 dwords are preloaded into SGPRs at wave launch), the output last.
 __global__ __launch_bounds__(NW * WAVE) void q4_gemv_block_kernel(const uint32_t *Wt, const uint16_t *St, const uint16_t *Zt,
-                                                             const uint16_t *x, int xs, int M, int K, int N, int KS_,
+                                                             const uint16_t *x, int xs, int M, int K_, int N, int KS_,
                                                              int SUB_, void *__restrict__ y, int ys, int y_bf16,
                                                              int accumulate, int n_lo) {
     // KSNW: one subtile per item, split over all NW waves, each wave exactly
@@ -52,6 +52,7 @@ __global__ __launch_bounds__(NW * WAVE) void q4_gemv_block_kernel(const uint32_t
     const int KS = KSNW ? NW : KS_, SUB = KSNW ? 1 : SUB_;
     extern __shared__ __align__(16) unsigned char smem[];
     constexpr int GW = DENSE_GW;
+    const int K = KSNW ? NW * GW * QGROUP : K_;
     const int G = KSNW ? NW * GW : K / QGROUP, kc = x_row_stride(K), nsub = (N + 15) / 16, gpk = KSNW ? GW : dense_gpk(G),
               items = (nsub + SUB - 1) / SUB;
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid / WAVE), lane = tid % WAVE,
@@ -66,7 +67,8 @@ __global__ __launch_bounds__(NW * WAVE) void q4_gemv_block_kernel(const uint32_t
     // read)
     XRegs xv;
     if constexpr (XPT > 0) stage_regs_issue<XPT>(x, xs, M, K, xv);
-    else stage_x_issue(x, xs, M, K, xl);
+    else
+        stage_rows_issue([&](int m) { return x + int64_t(m) * xs; }, M, K, xl, KSNW ? NW : int(blockDim.x) / WAVE);
     __builtin_amdgcn_sched_barrier(0);  // every activation load goes out before the weight loads
     WaveRange<GW, HAS_Z, true> wr[1];
     wr[0].fetch(tile_of(blockIdx.x), g0, min(ng, GW), lane);

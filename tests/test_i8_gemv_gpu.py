@@ -70,6 +70,35 @@ def test_i8_gemv_grouped_rows(gpu, oracle, group, M):
         assert rel_err(y, oracle.i8_linear_f64(W8, S, x16, M, xs=HC * SH, rpg=rpg, group=group)) <= TOL
 
 
+@pytest.mark.parametrize("group", [32, 16])
+@pytest.mark.parametrize("N,K,M", [(16, 128, 1), (20, 384, 9), (4097, 1152, 4), (8200, 256, 15), (8200, 1152, 17),
+                                   (8193, 128, 5), (12289, 640, 16), (12300, 1152, 32), (16400, 2176, 29),
+                                   (300, 192, 11)])
+def test_i8_gemv_streamed(gpu, group, N, K, M):
+    """The streamed kernel's shapes (1 to 4 row tiles per block, one and two row blocks,
+    K parts of unequal and zero groups, ragged rows and tiles), fp16 rows between wider
+    ones, fp32 and bf16 results and accumulation. Integer activations and power-of-two
+    scales: partial sums are exact fp32 integers times 2^-3, so results are bit-exact."""
+    import torch
+    print(f"i8 gemv streamed group={group} N={N} K={K} M={M}", flush=True)
+    rng = np.random.default_rng(N + K + M)
+    W8 = rng.integers(-128, 128, size=(N, K), dtype=np.int8)
+    S = np.ldexp(1.0, rng.integers(-3, 2, size=(N, K // group))).astype(np.float32)
+    x = np.full((M, K + 8), np.nan, np.float16)
+    x[:, :K] = rng.integers(-4, 5, size=(M, K))
+    xi = x[:, :K].astype(np.float64)
+    ref = xi @ (W8.astype(np.float64) * np.repeat(S, group, axis=1)).T
+    y = torch.full((M, N + 3), 2.0, dtype=torch.float32, device=gpu)
+    Wt, St = qwq4.i8_tile(to_dev(W8, gpu), to_dev(S, gpu), group)
+    xd = to_dev(x.view(np.uint16), gpu)
+    qwq4.gemv_i8(Wt, St, N, K, xd, M, group=group, y=y, accumulate=True, xs=K + 8, ys=N + 3)
+    yh = host(y)
+    assert np.all(yh[:, N:] == 2.0)
+    assert np.array_equal(yh[:, :N], (ref + 2.0).astype(np.float32))
+    yb = host(qwq4.gemv_i8(Wt, St, N, K, xd, M, group=group, xs=K + 8, y_bf16=True))
+    assert bf16_err_ok(yb, ref)
+
+
 def test_i8_gemv_rows_independent(gpu, oracle):
     """A token row's result does not depend on the batch it is in (bit for bit)."""
     N, K = 1000, 4096

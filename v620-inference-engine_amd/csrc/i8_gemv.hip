@@ -190,6 +190,179 @@ __global__ __launch_bounds__(I8_MAX_KS *WAVE) void i8_gemv_kernel(const uint4 *W
     if (kp == 0) store_rows<MB, MR>(acc[0], y, ys, y_bf16, accumulate, M, N, blockIdx.x, lane);
 }
 
+// ------------------------------------------------------------ rows streamed
+// The kernel above stages every activation row of the whole K per 16 weight
+// rows: 8 KB a row of 4096 against 64 KB of weights, so the copy outweighs the
+// weights from 8 rows on, nothing is requested while it is waited for, and past
+// 16 rows of 4096 (9 of 6144) the batch no longer fits LDS and runs as several
+// launches. Here a block takes 16 NS weight rows and moves the rows' K in
+// groups of 128 through a double buffer: its 8 waves split K, each widens a
+// weight once for 16 MB rows, and the next group's rows (direct global -> LDS
+// loads), weights and scales (registers) are requested before a group is
+// computed. The parts are added through LDS in part order. Products, the
+// fp32 sum per scale group and its scaling are those above. K a multiple of
+// 128, no row slices. Bound by the weight stream; before -> after, groups of
+// 32, us: 6144->4096 at 1 / 3 / 16 / 32 rows 9.1 / 10.0 / 20.3 / 31.0 -> 7.2 /
+// 7.1 / 8.0 / 12.1, 4096->12288 12.1 / 12.9 / 21.4 / 42.1 -> 11.6 / 11.7 /
+// 13.0 / 15.6 (3.9-4.9 TB/s at 3 rows).
+template <int MB, int NS>
+struct I8Wide {
+    static constexpr int WK = 8, ROWS = 16 * NS, BM = 16 * MB;
+    static constexpr int A = WK * BM * 256;      // bytes of a group's rows
+    static constexpr int SLOT = 16 * ROWS * 4;   // closing sums: 16 rows at a time per wave
+    static_assert(A >= 4 * SLOT, "four slots in each buffer");
+};
+
+// 8-byte half h (0..31) of row r of a part's tile [16 MB][128]
+__device__ __forceinline__ int i8w_at(int r, int h) { return r * 256 + (((h >> 1) ^ (r & 15)) << 4) + (h & 1) * 8; }
+
+template <int GRP, int MB, int NS>
+__device__ __forceinline__ void i8_wide_block(const uint4 *Wt, const float *St, const uint16_t *__restrict__ x, int xs,
+                                              int M, int K, int N, void *__restrict__ y, int ys, int y_bf16,
+                                              int accumulate) {
+    using S = I8Wide<MB, NS>;
+    constexpr int WK = S::WK, SPS = 64 / GRP;
+    __shared__ __align__(16) unsigned char a0[S::A], a1[S::A];
+    typedef float sv_t __attribute__((ext_vector_type(SPS)));
+    const int tid = threadIdx.x, wk = __builtin_amdgcn_readfirstlane(tid / WAVE), lane = tid % WAVE, n = lane % 16,
+              q = lane / 16;
+    const int nb = int(gridDim.x), xq = nb / 8, xr = nb % 8, xcd = int(blockIdx.x) % 8;
+    const int item = xcd * xq + min(xcd, xr) + int(blockIdx.x) / 8;  // a contiguous range of row blocks per XCD
+    const int nsub = (N + 15) / 16, steps = K / 64;
+    const int G = K / 128, per = G / WK, rem = G % WK;
+    const int g0 = wk * per + min(wk, rem), ng = per + (wk < rem), ngmax = per + (rem > 0);
+    const uint4 *w[NS];
+    const sv_t *sc[NS];
+#pragma unroll
+    for (int j = 0; j < NS; ++j) {
+        const int64_t sub = min(item * NS + j, nsub - 1);
+        w[j] = Wt + sub * steps * WAVE;
+        sc[j] = reinterpret_cast<const sv_t *>(St) + sub * steps * 16;
+    }
+    int xo[4 * MB];  // instruction j moves rows 4 j .. 4 j + 3 of the part
+#pragma unroll
+    for (int j = 0; j < 4 * MB; ++j) {
+        const int r = j * 4 + q;
+        xo[j] = min(r, M - 1) * xs + ((n ^ (r & 15)) * 8);
+    }
+    struct WR {
+        uint4 w[NS][2];
+        sv_t s[NS][2];
+    };
+    auto issue = [&](int i, unsigned char *dst, WR &r) {
+        const int g = min(g0 + min(i, max(ng, 1) - 1), G - 1);  // past the end: a valid (unused) one
+#pragma unroll
+        for (int j = 0; j < 4 * MB; ++j)
+            if (4 * j < M)  // (uniform)
+                __builtin_amdgcn_global_load_lds(x + g * 128 + xo[j], dst + wk * (S::BM * 256) + j * 1024, 16, 0, 0);
+#pragma unroll
+        for (int j = 0; j < NS; ++j)
+#pragma unroll
+            for (int t = 0; t < 2; ++t) {
+                r.w[j][t] = w[j][(2 * g + t) * WAVE + lane];
+                r.s[j][t] = sc[j][(2 * g + t) * 16 + n];
+            }
+    };
+    int ar[MB];  // rows past M read the last one
+#pragma unroll
+    for (int mb = 0; mb < MB; ++mb) ar[mb] = min(mb * 16 + n, M - 1);
+    f32x4 acc[NS][MB];
+    const f32x4 zero = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int j = 0; j < NS; ++j)
+#pragma unroll
+        for (int mb = 0; mb < MB; ++mb) acc[j][mb] = zero;
+    auto compute = [&](const unsigned char *ab, const WR &r) {
+        const unsigned char *a = ab + wk * (S::BM * 256);
+#pragma unroll
+        for (int t = 0; t < 2; ++t) {
+            if constexpr (GRP == 32) {
+                uint4 fa[MB], fb[MB];
+#pragma unroll
+                for (int mb = 0; mb < MB; ++mb) {
+                    fa[mb] = *reinterpret_cast<const uint4 *>(a + i8w_at(ar[mb], 2 * (8 * t + q)));
+                    fb[mb] = *reinterpret_cast<const uint4 *>(a + i8w_at(ar[mb], 2 * (8 * t + 4 + q)));
+                }
+#pragma unroll
+                for (int j = 0; j < NS; ++j) {
+                    const uint4 &v = r.w[j][t];
+                    const uint4 wa = i8x8_to_f16x8(v.x, v.y), wb = i8x8_to_f16x8(v.z, v.w);
+#pragma unroll
+                    for (int mb = 0; mb < MB; ++mb) {
+                        const f32x4 ra = mfma16<F16>(fa[mb], wa, zero), rb = mfma16<F16>(fb[mb], wb, zero);
+                        acc[j][mb] += r.s[j][t][0] * ra + r.s[j][t][1] * rb;
+                    }
+                }
+            } else {
+                uint2 f[MB][4];
+#pragma unroll
+                for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+                    for (int g = 0; g < 4; ++g)
+                        f[mb][g] = *reinterpret_cast<const uint2 *>(a + i8w_at(ar[mb], 16 * t + 4 * g + q));
+#pragma unroll
+                for (int j = 0; j < NS; ++j) {
+                    const uint32_t v[4] = {r.w[j][t].x, r.w[j][t].y, r.w[j][t].z, r.w[j][t].w};
+#pragma unroll
+                    for (int g = 0; g < 4; ++g) {
+                        const uint2 wg = i8x4_to_f16x4(v[g]);
+#pragma unroll
+                        for (int mb = 0; mb < MB; ++mb) acc[j][mb] += r.s[j][t][g] * mfma16x16(f[mb][g], wg, zero);
+                    }
+                }
+            }
+        }
+    };
+    WR w0, w1;
+    issue(0, a0, w0);
+    // a part's rows are written and read by one wave: the wait for its own loads
+    // suffices for them, and the reads of the buffer being refilled are complete
+    auto step = [&](int i, const unsigned char *a, WR &cur, unsigned char *an, WR &next) {
+        __builtin_amdgcn_sched_barrier(0);
+        wait_vm_below<0>();
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_sched_barrier(0);
+        issue(i + 1, an, next);
+        __builtin_amdgcn_sched_barrier(0);
+        if (i < ng) compute(a, cur);
+    };
+    int i = 0;
+    for (; i + 2 <= ngmax; i += 2) {
+        step(i, a0, w0, a1, w1);
+        step(i + 1, a1, w1, a0, w0);
+    }
+    if (i < ngmax) step(i, a0, w0, a1, w1);
+    wait_vm_below<0>();
+
+    // 16 rows at a time: the wave's sums to its slot ([row][weight rows]), then
+    // each element's parts are added in part order
+    auto slot = [&](int k) { return reinterpret_cast<float *>((k < 4 ? a0 : a1) + (k % 4) * S::SLOT); };
+#pragma unroll
+    for (int mb = 0; mb < MB; ++mb) {
+        lds_barrier();
+        float *mine = slot(wk);
+#pragma unroll
+        for (int j = 0; j < NS; ++j)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) mine[(4 * q + r) * S::ROWS + 16 * j + n] = acc[j][mb][r];
+        lds_barrier();
+        for (int c = tid; c < 16 * S::ROWS; c += 512) {
+            const int col = c % S::ROWS, tr = c / S::ROWS, m = mb * 16 + tr, row = item * S::ROWS + col;
+            float v = 0.f;
+#pragma unroll
+            for (int k = 0; k < WK; ++k) v += slot(k)[tr * S::ROWS + col];
+            if (m < M && row < N) store_y(y, int64_t(m) * ys + row, v, y_bf16, accumulate);
+        }
+    }
+}
+
+template <int GRP, int MB, int NS>
+__global__ __launch_bounds__(512, (MB == 1 && NS <= 2 ? 4 : 2)) void i8_wide_kernel(
+    const uint4 *Wt, const float *St, const uint16_t *x, int xs, int M, int K, int N, void *__restrict__ y, int ys,
+    int y_bf16, int accumulate) {
+    i8_wide_block<GRP, MB, NS>(Wt, St, x, xs, M, K, N, y, ys, y_bf16, accumulate);
+}
+
 // ------------------------------------------------------------ tiled format
 // Wt uint4 [ceil(N/16)][K/64][64]: entry (tile, s, lane l) holds 16 int8
 // weights of row 16 tile + l % 16, q = l / 16, of the 64-element step s:
@@ -289,9 +462,56 @@ static void launch_i8_fit(const I8Args &a, hipStream_t s) {
 
 bool i8_fits(int M, int K, int N, int group, int rpg) { return i8_lds_bytes(M, K, N, group, rpg) <= 160 * 1024; }
 
+template <int GRP, int MB, int NS>
+static void launch_i8_wide_t(const I8Args &a, hipStream_t s) {
+    constexpr int R = I8Wide<MB, NS>::ROWS;
+    i8_wide_kernel<GRP, MB, NS><<<unsigned((a.N + R - 1) / R), 512, 0, s>>>(a.W, a.S, a.x, a.xs, a.M, a.K, a.N, a.y,
+                                                                            a.ys, a.y_bf16, a.accumulate);
+}
+
+// Row tiles per block: the fewest that make one round of a block per CU
+// (4096->12288, 768 tiles, at 16 rows 16.1 / 15.3 / 13.0 / 14.3 us with 1 / 2 / 3
+// / 4; 3072->6144, 384 tiles, 7.6 / 6.6 / 8.0 / 9.1; 6144->4096, 256 tiles, 8.0 /
+// 9.6 / 12.1 / 14.4). Beyond three rounds of single tiles 2 up to 16 rows, where
+// two blocks share a CU, and 4 above (2048->32000 18.6 against 18.7-23.5, and
+// 24.1 against 28.5-40.7).
+template <int GRP>
+static void launch_i8_wide(const I8Args &a, hipStream_t s) {
+    const int ns = ((a.N + 15) / 16 + 255) / 256;
+    if (a.M <= 16) {
+        if (ns == 1) launch_i8_wide_t<GRP, 1, 1>(a, s);
+        else if (ns == 3) launch_i8_wide_t<GRP, 1, 3>(a, s);
+        else launch_i8_wide_t<GRP, 1, 2>(a, s);
+    } else {
+        if (ns == 1) launch_i8_wide_t<GRP, 2, 1>(a, s);
+        else if (ns == 2) launch_i8_wide_t<GRP, 2, 2>(a, s);
+        else if (ns == 3) launch_i8_wide_t<GRP, 2, 3>(a, s);
+        else launch_i8_wide_t<GRP, 2, 4>(a, s);
+    }
+}
+
+// The streamed kernel takes every batch where its blocks are one round of the
+// CUs, and batches above 8 beyond. Up to 8 rows of more than 768 tiles the
+// staged kernel's small blocks keep more of the weight stream in flight
+// (2048->32000 at 1 / 8 / 16 rows 14.0 / 16.9 / 22.9 us against 15.8 / 16.8 /
+// 18.6), as with groups of 16 (a quarter more bytes and twice the MFMAs) up to 4 rows of
+// more than 640 tiles (4096->12288 at 1 / 3 / 8 rows 13.1 / 13.7 / 21.4 against 14.1 /
+// 14.2 / 14.2; 2560->10000, 625 tiles, 9.3 / 9.8 / 11.8 against 9.0 / 9.2 / 9.6).
+// xs: 32-bit row offsets.
+static bool i8_wide(const I8Args &a) {
+    const int nt = (a.N + 15) / 16;
+    if (a.rpg != 0 || a.K % 128 != 0 || a.xs > 1 << 25) return false;
+    if (a.M > 8) return true;
+    return nt <= 768 && !(a.group == 16 && a.M <= 4 && nt > 640);
+}
+
 // Batches whose activations exceed LDS run as several launches of fewer rows
 // (the caller has checked that one row fits).
 void launch_i8_gemv(const I8Args &a, hipStream_t s) {
+    if (i8_wide(a)) {
+        a.group == 32 ? launch_i8_wide<32>(a, s) : launch_i8_wide<16>(a, s);
+        return;
+    }
     if (i8_fits(a.M, a.K, a.N, a.group, a.rpg)) {
         launch_i8_fit(a, s);
         return;

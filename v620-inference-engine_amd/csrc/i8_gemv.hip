@@ -201,10 +201,11 @@ __global__ __launch_bounds__(I8_MAX_KS *WAVE) void i8_gemv_kernel(const uint4 *W
 // loads), weights and scales (registers) are requested before a group is
 // computed. The parts are added through LDS in part order. Products, the
 // fp32 sum per scale group and its scaling are those above. K a multiple of
-// 128, no row slices. Bound by the weight stream; before -> after, groups of
-// 32, us: 6144->4096 at 1 / 3 / 16 / 32 rows 9.1 / 10.0 / 20.3 / 31.0 -> 7.2 /
-// 7.1 / 8.0 / 12.1, 4096->12288 12.1 / 12.9 / 21.4 / 42.1 -> 11.6 / 11.7 /
-// 13.0 / 15.6 (3.9-4.9 TB/s at 3 rows).
+// 128, no row slices. Bound by the weight stream, which is read non-temporal
+// and in block order (cached and in a range per XCD: 7% slower at 4096->12288).
+// Before -> after on 1.2 GB of weights, groups of 32, us: 6144->4096 at 1 / 4 /
+// 8 / 16 rows 8.8 / 9.7 / 10.2 / 19.7 -> 7.4 / 7.3 / 7.6 / 8.9, 4096->12288 12.2 /
+// 13.2 / 15.1 / 21.9 -> 12.2 / 12.2 / 12.4 / 13.7 (4.6 TB/s at 4 rows).
 template <int MB, int NS>
 struct I8Wide {
     static constexpr int WK = 8, ROWS = 16 * NS, BM = 16 * MB;
@@ -222,12 +223,12 @@ __device__ __forceinline__ void i8_wide_block(const uint4 *Wt, const float *St, 
                                               int accumulate) {
     using S = I8Wide<MB, NS>;
     constexpr int WK = S::WK, SPS = 64 / GRP;
+    typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
     __shared__ __align__(16) unsigned char a0[S::A], a1[S::A];
     typedef float sv_t __attribute__((ext_vector_type(SPS)));
     const int tid = threadIdx.x, wk = __builtin_amdgcn_readfirstlane(tid / WAVE), lane = tid % WAVE, n = lane % 16,
               q = lane / 16;
-    const int nb = int(gridDim.x), xq = nb / 8, xr = nb % 8, xcd = int(blockIdx.x) % 8;
-    const int item = xcd * xq + min(xcd, xr) + int(blockIdx.x) / 8;  // a contiguous range of row blocks per XCD
+    const int item = int(blockIdx.x);
     const int nsub = (N + 15) / 16, steps = K / 64;
     const int G = K / 128, per = G / WK, rem = G % WK;
     const int g0 = wk * per + min(wk, rem), ng = per + (wk < rem), ngmax = per + (rem > 0);
@@ -259,7 +260,8 @@ __device__ __forceinline__ void i8_wide_block(const uint4 *Wt, const float *St, 
         for (int j = 0; j < NS; ++j)
 #pragma unroll
             for (int t = 0; t < 2; ++t) {
-                r.w[j][t] = w[j][(2 * g + t) * WAVE + lane];
+                const u32x4 v = __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(w[j] + (2 * g + t) * WAVE + lane));
+                r.w[j][t] = make_uint4(v[0], v[1], v[2], v[3]);
                 r.s[j][t] = sc[j][(2 * g + t) * 16 + n];
             }
     };
@@ -303,12 +305,21 @@ __device__ __forceinline__ void i8_wide_block(const uint4 *Wt, const float *St, 
 #pragma unroll
                 for (int j = 0; j < NS; ++j) {
                     const uint32_t v[4] = {r.w[j][t].x, r.w[j][t].y, r.w[j][t].z, r.w[j][t].w};
+                    // the step's four groups first, so that the long sum has one
+                    // term per step as with groups of 32 (and 8 parts are no less
+                    // exact than the staged kernel's 16)
+                    f32x4 p[MB];
 #pragma unroll
                     for (int g = 0; g < 4; ++g) {
                         const uint2 wg = i8x4_to_f16x4(v[g]);
 #pragma unroll
-                        for (int mb = 0; mb < MB; ++mb) acc[j][mb] += r.s[j][t][g] * mfma16x16(f[mb][g], wg, zero);
+                        for (int mb = 0; mb < MB; ++mb) {
+                            const f32x4 rg = mfma16x16(f[mb][g], wg, zero);
+                            p[mb] = g == 0 ? r.s[j][t][g] * rg : p[mb] + r.s[j][t][g] * rg;
+                        }
                     }
+#pragma unroll
+                    for (int mb = 0; mb < MB; ++mb) acc[j][mb] += p[mb];
                 }
             }
         }
@@ -494,15 +505,16 @@ static void launch_i8_wide(const I8Args &a, hipStream_t s) {
 // CUs, and batches above 8 beyond. Up to 8 rows of more than 768 tiles the
 // staged kernel's small blocks keep more of the weight stream in flight
 // (2048->32000 at 1 / 8 / 16 rows 14.0 / 16.9 / 22.9 us against 15.8 / 16.8 /
-// 18.6), as with groups of 16 (a quarter more bytes and twice the MFMAs) up to 4 rows of
-// more than 640 tiles (4096->12288 at 1 / 3 / 8 rows 13.1 / 13.7 / 21.4 against 14.1 /
-// 14.2 / 14.2; 2560->10000, 625 tiles, 9.3 / 9.8 / 11.8 against 9.0 / 9.2 / 9.6).
+// 18.6), as with groups of 16 (a quarter more bytes and twice the MFMAs) for one
+// row of more than 640 tiles (4096->12288 at 1 / 2 / 4 rows 13.1 / 13.6 / 15.2
+// against 14.0 / 13.5 / 13.7; 2560->10000, 625 tiles, 9.1 / 9.2 / 10.1 against
+// 8.1 / 8.1 / 8.3).
 // xs: 32-bit row offsets.
 static bool i8_wide(const I8Args &a) {
     const int nt = (a.N + 15) / 16;
     if (a.rpg != 0 || a.K % 128 != 0 || a.xs > 1 << 25) return false;
     if (a.M > 8) return true;
-    return nt <= 768 && !(a.group == 16 && a.M <= 4 && nt > 640);
+    return nt <= 768 && !(a.group == 16 && a.M == 1 && nt > 640);
 }
 
 // Batches whose activations exceed LDS run as several launches of fewer rows

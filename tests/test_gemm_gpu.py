@@ -282,11 +282,16 @@ def test_gemm_ksplit_nonfinite(gpu, oracle):
     assert rel_err(Y[ok], oracle.q4_linear(W, S, Z, N, K, x[ok].astype(np.float32))) <= TOL
 
 
+def _light_load(T, k, E, H, F):
+    """The grouped GEMMs' choice of the 32-slot kernels (light_load, moe_grouped.hip)."""
+    return T * k <= 7 * E and -(-F // 256) * E * 4096 // H >= 320
+
+
 # Few tokens per expert on average (the 32-slot kernels), with loads around
 # the block sizes: experts of 1, 16, 17, 32, 33 and over 160 tokens beside
 # empty ones; F and H off the 256- and 512-row blocks, an odd number of K groups.
 @pytest.mark.parametrize("yp16", [False, True])
-@pytest.mark.parametrize("E,H,F,zeros", [(96, 384, 640, True), (64, 640, 128, False), (128, 512, 384, True)])
+@pytest.mark.parametrize("E,H,F,zeros", [(96, 384, 640, True), (80, 640, 128, False), (128, 512, 384, True)])
 def test_grouped_light_loads(gpu, oracle, E, H, F, zeros, yp16):
     print(f"grouped light E={E} H={H} F={F} zeros={zeros} yp16={yp16}", flush=True)
     want = {3: 1, 5: 16, 9: 17, 20: 32, 33: 33, 50: 170, E - 1: 5}
@@ -301,8 +306,36 @@ def test_grouped_light_loads(gpu, oracle, E, H, F, zeros, yp16):
     out, h_ref, yp_ref = oracle.moe(xf, l, k, *ex, want_parts=True)
     from test_moe_gpu import _experts_dev
     (dg, du, dd), E, F = _experts_dev(gpu, ex)
+    assert _light_load(T, k, E, H, F)
     r = qwq4.moe_route(to_dev(l, gpu), k, tile_m=qwq4.moe_grouped_tile_m())
     h, yp = qwq4.moe_experts_grouped(dg, du, dd, r, to_dev(xb, gpu), E, F, yp_f16=yp16)
     assert rel_err(host(h).astype(np.float32), h_ref) <= TOL
     assert rel_err(host(yp).astype(np.float32), yp_ref) <= TOL
     assert rel_err(host(qwq4.moe_combine(yp, r, H, out_bf16=False)), out) <= TOL
+
+
+# A chunk of few tokens per expert (the 32-slot kernels) and one of many (tiles
+# of 32 to 160 slots) that begins with the same rows; experts of under and over
+# 32 tokens, F and H off the 256- and 512-row blocks, an odd number of K groups.
+@pytest.mark.parametrize("E,H,F,zeros,yp16", [(64, 640, 384, True, True), (64, 1152, 640, False, False)])
+def test_grouped_rows_independent(gpu, E, H, F, zeros, yp16):
+    """A token's expert rows do not depend on the length of its chunk: h, the
+    experts' outputs and the combined rows equal, bit for bit."""
+    import torch
+    k, T0, T1 = 4, 90, 1500
+    print(f"grouped rows E={E} H={H} F={F} zeros={zeros}", flush=True)
+    l = np.random.default_rng(E + F).standard_normal((T1, E)).astype(np.float32)
+    l[:40, 11] += 8.0  # one expert of over 32 of the short chunk's tokens
+    ex = synth.experts(64, E, H, F, zeros=zeros)
+    xb, _ = synth.acts(64, f"li{H}", T1, H)
+    from test_moe_gpu import _experts_dev
+    (dg, du, dd), E, F = _experts_dev(gpu, ex)
+    assert _light_load(T0, k, E, H, F) and not _light_load(T1, k, E, H, F)
+    got = []
+    for T in (T0, T1):
+        r = qwq4.moe_route(to_dev(l[:T], gpu), k, tile_m=qwq4.moe_grouped_tile_m())
+        h, yp = qwq4.moe_experts_grouped(dg, du, dd, r, to_dev(xb[:T], gpu), E, F, yp_f16=yp16)
+        slots = r.tok_slot[:T0].long()
+        got.append([h[slots], yp[slots], qwq4.moe_combine(yp, r, H, out_bf16=False)[:T0]])
+    for a, b in zip(*got):
+        assert torch.equal(a, b)

@@ -157,38 +157,37 @@ __global__ __launch_bounds__(G_THREADS) void moe_down_gemm_kernel(
 
 // ---- chunks with few tokens per expert: 32 slots by 512 weight rows, bound
 // by the weight stream
-// A wave holds 64 weight rows (four 16-row subtiles) and every slot of the
-// block, so each weight is read and unpacked once per 32 slots. What the
-// stream needs is requests in flight and few instructions per weight:
-//   - the 16x16x32 MFMA takes a subtile's entries as they lie (1 KB of
-//     contiguous weights per wave load) and up to 16 slots cost half the
-//     matrix time of the 32-row one;
-//   - operands are the exact q - z (10 VALU instructions per 8 weights
-//     instead of 15), the scale is applied to the group's fp32 sum;
-//   - with 16 or 32 accumulator registers a wave fits 128 VGPRs, so a CU
-//     holds two blocks, each wave a whole group (128 K) ahead. A group's A
-//     rows are 8 KB, one direct load per wave.
+// A wave holds 64 weight rows (two 32-row groups, as gemm_tile_rd2) and every
+// slot of the block, so each weight is read and dequantised once per 32 slots.
+// What the stream needs is requests in flight: with 32 accumulator registers a
+// wave fits 128 VGPRs, so a CU holds two blocks (of the taller tiles one), each
+// wave a whole group (128 K) ahead; a group's A rows are 8 KB, one direct load
+// per wave. Operands, MFMA and K order are gemm_tile_rd2's, so a slot's sums
+// are the same bits in a chunk of any length.
 constexpr int LIGHT_A = 32 * 256;  // bytes of a group's A: [32][128] fp16
 
-// 16-byte chunk c (0..15) of row r of the A tile: the fragment reads take 16
-// rows at one chunk of each 64-byte quarter
+// 16-byte chunk c (0..15) of row r of the A tile: a fragment read takes 32
+// rows at one chunk of each 128-byte half
 __device__ __forceinline__ int light_swz(int r, int c) { return r * 256 + ((c ^ (r & 15)) << 4); }
 
-// The wave's four subtiles' entries (w[j] + lane's, 64 per group) and its own
-// row's scale and zero word (bs: row = lane).
-struct LightW {
-    const uint4 *w[4];
-};
+// dequant8's values, with one VALU instruction less: q - z exact, then the
+// rounding multiply. zl: -(1024 + z), zh: -(64 + z).
+__device__ __forceinline__ uint4 dequant8_light(uint32_t w, h2 zl, h2 zh, h2 s2) {
+    const uint4 d = unpack8_exact(w, zl, zh);
+    auto mul = [&](uint32_t v) { return __builtin_bit_cast(uint32_t, __builtin_bit_cast(h2, v) * s2); };
+    return make_uint4(mul(d.x), mul(d.y), mul(d.z), mul(d.w));
+}
 
-// acc[j][mb] += the tile's 16-slot blocks mb (A rows arow, this lane's of the
-// loads) times subtile j's rows over all G groups
-template <int MB, bool HAS_Z, int USE>
-__device__ __forceinline__ void gemm_tile_light(const uint16_t *arow, const LightW &lw, const BRow &bs, int G, int lane,
-                                                f32x4 (&acc)[4][MB]) {
+// acc[j] += the tile's 32 slots (A rows arow, this lane's of the loads) times
+// row group j's rows (b0, b1: row lane % 32) over all G groups; bs: the lane's
+// own row (its scales and zeros).
+template <bool HAS_Z, int USE>
+__device__ __forceinline__ void gemm_tile_light(const uint16_t *arow, const BRow &b0, const BRow &b1, const BRow &bs,
+                                                int G, int lane, f32x16 (&acc)[2]) {
     __shared__ __align__(16) unsigned char a0[LIGHT_A], a1[LIGHT_A];
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE), n = lane % 16, q = lane / 16;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE), l32 = lane % 32, lh = lane / 32;
     struct WR {
-        uint4 w[4];
+        uint4 w0[2], w1[2];  // 64-K halves of the group
         uint16_t s;
         uint32_t z;
     };
@@ -198,51 +197,33 @@ __device__ __forceinline__ void gemm_tile_light(const uint16_t *arow, const Ligh
         g = min(g, G - 1);  // past the end: a valid (unused) one
         __builtin_amdgcn_global_load_lds(arow + g * QGROUP + ac, dst + wave * 1024, 16, 0, 0);
 #pragma unroll
-        for (int j = 0; j < 4; ++j) r.w[j] = lw.w[j][g * 64 + lane];
+        for (int h = 0; h < 2; ++h) {
+            r.w0[h] = b0.w[g * 64 + (h * 2 + lh) * 16];
+            r.w1[h] = b1.w[g * 64 + (h * 2 + lh) * 16];
+        }
         r.s = bs.s[(g >> 2) * 64 + (g & 3)];
         if constexpr (HAS_Z) r.z = bs.z[(g >> 2) * 8];
     };
     auto compute = [&](const unsigned char *a, const WR &r, int g) {
-        uint32_t s = r.s, z = HAS_Z ? r.z : 0u, sv[4], zv[4];
+        uint32_t s = r.s, z = HAS_Z ? r.z : 0u, sv[2], zv[2] = {8u, 8u};
         asm volatile("" : "+v"(s), "+v"(z));  // taken here, not at their loads
-        split_quarters(s, sv);
-        if constexpr (HAS_Z) split_quarters((z >> (bs.zs + 4 * (g & 3))) & 0xfu, zv);
-        else zv[0] = zv[1] = zv[2] = zv[3] = 8u;
-        // two subtiles at a time, the fragments read again for the second two
-        // (held across all four they would cost MB 2 its registers)
+        split_halves(s * 0x10001u, sv[0], sv[1]);
+        if constexpr (HAS_Z) split_halves(((z >> (bs.zs + 4 * (g & 3))) & 0xfu) * 0x10001u, zv[0], zv[1]);
+        else zv[0] = zv[1] = 0x80008u;
+        h2 zl[2], zh[2], s2[2];
 #pragma unroll
-        for (int jp = 0; jp < 4; jp += 2) {
-            asm volatile("" ::: "memory");
-            h2 zl[2], zh[2];
-            f32x4 p[2][MB];
+        for (int j = 0; j < 2; ++j) {
+            zl[j] = __builtin_bit_cast(h2, zv[j] | 0xe400e400u);         // -(1024 + z)
+            zh[j] = __builtin_bit_cast(h2, (zv[j] << 4) + 0xd400d400u);  // -(64 + z)
+            s2[j] = __builtin_bit_cast(h2, sv[j]);
+        }
 #pragma unroll
-            for (int j = 0; j < 2; ++j) {
-                zl[j] = __builtin_bit_cast(h2, zv[jp + j] * 0x10001u | 0xe400e400u);         // -(1024 + z)
-                zh[j] = __builtin_bit_cast(h2, (zv[jp + j] << 4) * 0x10001u + 0xd400d400u);  // -(64 + z)
-#pragma unroll
-                for (int mb = 0; mb < MB; ++mb) p[j][mb] = f32x4{0.f, 0.f, 0.f, 0.f};
-            }
-#pragma unroll
-            for (int t = 0; t < 4; ++t) {
-                uint4 af[MB];
-#pragma unroll
-                for (int mb = 0; mb < MB; ++mb)
-                    af[mb] = *reinterpret_cast<const uint4 *>(a + light_swz(mb * 16 + n, q * 4 + t));
-#pragma unroll
-                for (int j = 0; j < 2; ++j) {
-                    const uint4 &w = r.w[jp + j];
-                    const uint4 f = unpack8_exact(t == 0 ? w.x : t == 1 ? w.y : t == 2 ? w.z : w.w, zl[j], zh[j]);
-#pragma unroll
-                    for (int mb = 0; mb < MB; ++mb) p[j][mb] = mfma16<F16>(af[mb], f, p[j][mb]);
-                }
-            }
-#pragma unroll
-            for (int j = 0; j < 2; ++j) {
-                const float sc = f16_bits_to_f32(uint16_t(sv[jp + j]));
-#pragma unroll
-                for (int mb = 0; mb < MB; ++mb) acc[jp + j][mb] += sc * p[j][mb];
-            }
-            __builtin_amdgcn_sched_barrier(0);
+        for (int t = 0; t < 8; ++t) {  // 16-K steps: 64-K half t / 4, word t % 4
+            const uint4 af = *reinterpret_cast<const uint4 *>(a + light_swz(l32, (t / 4) * 8 + t % 4 + 4 * lh));
+            const uint4 &w0 = r.w0[t / 4], &w1 = r.w1[t / 4];
+            auto word = [&](const uint4 &w) { return t % 4 == 0 ? w.x : t % 4 == 1 ? w.y : t % 4 == 2 ? w.z : w.w; };
+            acc[0] = mfma32<F16>(af, dequant8_light(word(w0), zl[0], zh[0], s2[0]), acc[0]);
+            acc[1] = mfma32<F16>(af, dequant8_light(word(w1), zl[1], zh[1], s2[1]), acc[1]);
         }
     };
     WR w0, w1;
@@ -268,8 +249,8 @@ __device__ __forceinline__ void gemm_tile_light(const uint16_t *arow, const Ligh
     __builtin_amdgcn_s_barrier();  // every wave is done with the buffers, and its loads into them have landed
 }
 
-// The lane index as a value the compiler cannot see through: per-lane
-// addresses are then formed again for each 32 slots, not held across them.
+// The lane index as a value the compiler cannot see through: the epilogue's
+// per-lane addresses are then formed after the loop, not held across it.
 __device__ __forceinline__ int light_lane() {
     int l = int(threadIdx.x) % WAVE;
     asm volatile("" : "+v"(l));
@@ -280,69 +261,47 @@ __device__ __forceinline__ int light_lane() {
 // 160 slots takes its z-th 32 slots. Entries above 32 are experts far above the
 // average; blocks past an entry's slots exit, after every first block.
 // gate/up: wave w holds the gate and the up rows of columns j0 + 32 w .. + 31
-// (subtiles 0, 1 and 2, 3), so h = silu(g) * u is formed in the wave.
-template <int MB, bool HAS_Z>
+// (groups 0 and 1), so h = silu(g) * u is formed in the wave.
+template <bool HAS_Z>
 __device__ __forceinline__ void gate_up_light(const GateUpTile &a, int e, int base, int mc) {
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE), lane = light_lane(), G = a.H / QGROUP;
     const int ar = min(wave * 4 + lane / 16, mc - 1), col0 = int(blockIdx.x) * 256 + wave * 32;
-    const int64_t sub0 = int64_t(e) * (a.F / 16);
-    LightW lw;
-#pragma unroll
-    for (int j = 0; j < 4; ++j)
-        lw.w[j] = reinterpret_cast<const uint4 *>(j < 2 ? a.gw : a.uw) +
-                  (sub0 + min(col0 / 16 + j % 2, a.F / 16 - 1)) * G * 64;
+    const int64_t wrow = int64_t(e) * a.F + min(col0 + lane % 32, a.F - 1);
+    const BRow bg(a.gw, a.gs, a.gz, wrow, G), bu(a.uw, a.us, a.uz, wrow, G);
     const bool up = lane >= 32;
-    const BRow bs(a.gw, up ? a.us : a.gs, up ? a.uz : a.gz, sub0 * 16 + min(col0 + lane % 32, a.F - 1), G);
-    f32x4 acc[4][MB];
+    const BRow bs(a.gw, up ? a.us : a.gs, up ? a.uz : a.gz, wrow, G);
+    f32x16 acc[2] = {};
+    gemm_tile_light<HAS_Z, 0>(a.xh + int64_t(a.pair_tok[base + ar]) * a.H, bg, bu, bs, G, lane, acc);
+    const int lo = light_lane(), c = col0 + lo % 32;
 #pragma unroll
-    for (int j = 0; j < 4; ++j)
-#pragma unroll
-        for (int mb = 0; mb < MB; ++mb) acc[j][mb] = f32x4{0.f, 0.f, 0.f, 0.f};
-    gemm_tile_light<MB, HAS_Z, 0>(a.xh + int64_t(a.pair_tok[base + ar]) * a.H, lw, bs, G, lane, acc);
-    const int lo = light_lane(), c = col0 + lo % 16;
-#pragma unroll
-    for (int mb = 0; mb < MB; ++mb)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const int m = mb * 16 + lo / 16 * 4 + r;
-#pragma unroll
-            for (int j = 0; j < 2; ++j)
-                if (m < mc && c + 16 * j < a.F)
-                    a.h[int64_t(base + m) * a.F + c + 16 * j] = f32_to_f16_sat(silu_mul(acc[j][mb][r], acc[2 + j][mb][r]));
-        }
+    for (int r = 0; r < 16; ++r) {
+        const int m = (r / 4) * 8 + lo / 32 * 4 + r % 4;
+        if (m < mc && c < a.F) a.h[int64_t(base + m) * a.F + c] = f32_to_f16_sat(silu_mul(acc[0][r], acc[1][r]));
+    }
 }
 
-template <int MB, bool HAS_Z, bool YP16>
+template <bool HAS_Z, bool YP16>
 __device__ __forceinline__ void down_light(const uint32_t *dw, const uint16_t *ds, const uint16_t *dz, int e, int base,
                                            int mc, const uint16_t *h, int H, int F, void *yp) {
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE), lane = light_lane(), G = F / QGROUP;
     const int ar = min(wave * 4 + lane / 16, mc - 1), n0 = int(blockIdx.x) * 512 + wave * 64;
-    const int64_t sub0 = int64_t(e) * (H / 16);
-    LightW lw;
+    const int64_t row0 = int64_t(e) * H;
+    const BRow b0(dw, ds, dz, row0 + min(n0 + lane % 32, H - 1), G),
+        b1(dw, ds, dz, row0 + min(n0 + 32 + lane % 32, H - 1), G), bs(dw, ds, dz, row0 + min(n0 + lane, H - 1), G);
+    f32x16 acc[2] = {};
+    gemm_tile_light<HAS_Z, 1 + YP16>(h + int64_t(base + ar) * F, b0, b1, bs, G, lane, acc);
+    const int lo = light_lane(), n = n0 + lo % 32;
 #pragma unroll
-    for (int j = 0; j < 4; ++j)
-        lw.w[j] = reinterpret_cast<const uint4 *>(dw) + (sub0 + min(n0 / 16 + j, H / 16 - 1)) * G * 64;
-    const BRow bs(dw, ds, dz, sub0 * 16 + min(n0 + lane, H - 1), G);
-    f32x4 acc[4][MB];
+    for (int r = 0; r < 16; ++r) {
+        const int m = (r / 4) * 8 + lo / 32 * 4 + r % 4;
+        const int64_t o = int64_t(base + m) * H + n;
 #pragma unroll
-    for (int j = 0; j < 4; ++j)
-#pragma unroll
-        for (int mb = 0; mb < MB; ++mb) acc[j][mb] = f32x4{0.f, 0.f, 0.f, 0.f};
-    gemm_tile_light<MB, HAS_Z, 1 + YP16>(h + int64_t(base + ar) * F, lw, bs, G, lane, acc);
-    const int lo = light_lane(), n = n0 + lo % 16;
-#pragma unroll
-    for (int mb = 0; mb < MB; ++mb)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const int m = mb * 16 + lo / 16 * 4 + r;
-            const int64_t o = int64_t(base + m) * H + n;
-#pragma unroll
-            for (int j = 0; j < 4; ++j)
-                if (m < mc && n + 16 * j < H) {
-                    if constexpr (YP16) static_cast<uint16_t *>(yp)[o + 16 * j] = f32_to_f16_sat(acc[j][mb][r]);
-                    else static_cast<float *>(yp)[o + 16 * j] = acc[j][mb][r];
-                }
-        }
+        for (int j = 0; j < 2; ++j)
+            if (m < mc && n + 32 * j < H) {
+                if constexpr (YP16) static_cast<uint16_t *>(yp)[o + 32 * j] = f32_to_f16_sat(acc[j][r]);
+                else static_cast<float *>(yp)[o + 32 * j] = acc[j][r];
+            }
+    }
 }
 
 template <bool HAS_Z>
@@ -357,8 +316,7 @@ __global__ __launch_bounds__(G_THREADS, 4) void moe_gate_up_light_kernel(GateUpT
     const int base = offsets[e] + m0, M = min(tile_rows(rem, GROUPED_TILE_M), rem);
     const int c0 = int(blockIdx.z) * 32;
     if (c0 >= M) return;
-    if (M - c0 <= 16) gate_up_light<1, HAS_Z>(a, e, base + c0, M - c0);
-    else gate_up_light<2, HAS_Z>(a, e, base + c0, min(32, M - c0));
+    gate_up_light<HAS_Z>(a, e, base + c0, min(32, M - c0));
 }
 
 template <bool HAS_Z, bool YP16>
@@ -372,22 +330,20 @@ __global__ __launch_bounds__(G_THREADS, 4) void moe_down_light_kernel(
     const int base = offsets[e] + m0, M = min(tile_rows(rem, GROUPED_TILE_M), rem);
     const int c0 = int(blockIdx.z) * 32;
     if (c0 >= M) return;
-    if (M - c0 <= 16) down_light<1, HAS_Z, YP16>(dw, ds, dz, e, base + c0, M - c0, h, H, F, yp);
-    else down_light<2, HAS_Z, YP16>(dw, ds, dz, e, base + c0, min(32, M - c0), h, H, F, yp);
+    down_light<HAS_Z, YP16>(dw, ds, dz, e, base + c0, min(32, M - c0), h, H, F, yp);
 }
 
-// Few tokens per expert on average: the light kernels, up to 20 where their
-// gate/up blocks fill the chip, fewer where they leave CUs with one block or
-// none (its groups then wait for their loads one by one; the longer K, the
-// more). Same box, both expert GEMMs, tiles of up to 160 slots against these:
-// 256 experts of 4096 / 1536, top 8, uneven loads, 2.5 tokens per expert
-// 446 -> 351 us, 7.8 533 -> 454, 19 655 -> 623, 28 725 -> 761; 128 experts of
-// 4096 / 1024 with zeros, 8 per expert 212 -> 191, 14 235 -> 241; 64 experts of
-// 4096 / 768, 4 per expert 84 -> 75, 8 97 -> 113; 64 of 2048 / 1408, 17 per
-// expert 98 -> 90.
+// Up to 7 tokens per expert on average: the light kernels, where their gate/up
+// blocks give most CUs two (elsewhere a block waits for its groups one by one;
+// the longer K, the more). Same box, both expert GEMMs, tiles of up to 160
+// slots against these: 256 experts of 4096 / 1536, top 8, uneven loads, 2
+// tokens per expert 408 -> 371 us, 5 468 -> 445; 256 of 2048 / 1152, 6.5 per
+// expert 223 -> 207; 128 of 4096 / 1024 with zeros, 5 per expert 190 -> 174; at 8
+// per expert gains and losses balance (256 of 3072 / 896 267 -> 275), at 19 they
+// lose 11%; 64 of 4096 / 768, 5 per expert 89 -> 93.
 static bool light_load(int T, int topk, int E, int H, int F) {
     const int64_t fill = int64_t((F + 255) / 256) * E * 4096 / H;  // gate/up blocks, at 4096 K
-    return int64_t(T) * topk <= (fill >= 640 ? 20 : fill >= 320 ? 12 : 6) * int64_t(E);
+    return int64_t(T) * topk <= int64_t(7) * E && fill >= 320;
 }
 
 void launch_moe_grouped(const MoeGroupedArgs &a, hipStream_t s) {
@@ -402,7 +358,9 @@ void launch_moe_grouped(const MoeGroupedArgs &a, hipStream_t s) {
     const dim3 g1(unsigned((a.F + 255) / 256), unsigned(max_tiles)), g2(unsigned((a.H + 511) / 512), unsigned(max_tiles));
     const GateUpTile gu{a.gw, a.uw, a.gs, a.gz, a.us, a.uz, a.pair_tok, xh, a.H, a.F, a.h};
     if (light_load(a.T, a.topk, a.E, a.H, a.F)) {
-        const dim3 l1(g1.x, g1.y, 5), l2(g2.x, g2.y, 5);
+        // (an entry has at most T slots)
+        const unsigned nz = unsigned(a.T < 160 ? (a.T + 31) / 32 : 5);
+        const dim3 l1(g1.x, g1.y, nz), l2(g2.x, g2.y, nz);
         auto gate_up = a.gz ? moe_gate_up_light_kernel<true> : moe_gate_up_light_kernel<false>;
         gate_up<<<l1, G_THREADS, 0, s>>>(gu, a.offsets, a.tile_e, a.tile_m0, a.n_tiles);
         auto down = a.dz ? (a.yp_f16 ? moe_down_light_kernel<true, true> : moe_down_light_kernel<true, false>)

@@ -110,6 +110,31 @@ def test_i8_gemv_rows_independent(gpu, oracle):
         assert np.array_equal(y1[0].view(np.uint32), y8[m].view(np.uint32))
 
 
+# Batches on both sides of every change of kernel: above 768 row tiles the staged
+# kernel up to 8 rows and the streamed one from 9, with groups of 16 and 641 to
+# 768 tiles the staged one for a single row, elsewhere one kernel with one or two
+# row blocks; whole K groups that divide into the parts, that do not, and fewer
+# than parts.
+@pytest.mark.parametrize("group", [32, 16])
+@pytest.mark.parametrize("N,K", [(12304, 2048), (12289, 1152), (12300, 384), (12288, 1664), (10256, 4096), (4096, 6144),
+                                 (1000, 896), (300, 192)])
+def test_i8_gemv_rows_independent_of_batch(gpu, group, N, K):
+    """A token row's result is the same bits in every batch of 1 to 32 rows."""
+    import torch
+    print(f"i8 rows independent group={group} N={N} K={K}", flush=True)
+    g = torch.Generator(device=gpu)
+    g.manual_seed(N + K)
+    W8 = torch.randint(-127, 128, (N, K), generator=g, device=gpu, dtype=torch.int32).to(torch.int8)
+    S = (torch.randn((N, K // group), generator=g, device=gpu) * 0.002).abs()
+    x = torch.randn((32, K), generator=g, device=gpu).to(torch.float16)
+    Wt, St = qwq4.i8_tile(W8, S, group)
+    y32 = qwq4.gemv_i8(Wt, St, N, K, x, 32, group=group)
+    for M in (1, 2, 3, 8, 9, 16, 17):
+        for m0 in {0, 32 - M}:
+            y = qwq4.gemv_i8(Wt, St, N, K, x[m0:m0 + M], M, group=group)
+            assert torch.equal(y.view(torch.int32), y32[m0:m0 + M].view(torch.int32)), (M, m0)
+
+
 def test_i8_gemv_strides_bf16_out_and_accumulate(gpu, oracle):
     import torch
     N, K, M = 500, 1024, 5

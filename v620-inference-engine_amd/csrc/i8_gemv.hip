@@ -56,6 +56,43 @@ __device__ __forceinline__ f32x4 mfma16x16(const uint2 &a, const uint2 &b, const
                                                  0);
 }
 
+// One 64-element step added to a sum: its groups' scaled products first
+// (step_mul, then fused), so that the long sum has one term per step. No
+// contraction but the fused ones written: both kernels below then give the same
+// bits.
+__device__ __forceinline__ float step_mul(float s, float r) {
+#pragma clang fp contract(off)
+    return s * r;
+}
+__device__ __forceinline__ float step_sum(float acc, float step) {
+#pragma clang fp contract(off)
+    return acc + step;
+}
+__device__ __forceinline__ float i8_add32(float acc, float s0, float r0, float s1, float r1) {
+    return step_sum(acc, __builtin_fmaf(s0, r0, step_mul(s1, r1)));
+}
+
+// K split. Ungrouped rows of a K of whole 128-element groups: up to 8 parts of
+// whole groups, the first ones a group longer where they do not divide, whatever
+// the batch and the matrix's rows, in both kernels below: a token row's result
+// does not depend on the batch it is in. Elsewhere (the staged kernel alone) KS
+// parts of equally many 64-element steps.
+__host__ __device__ inline bool i8_whole_groups(int K, int rpg) { return rpg == 0 && K % 128 == 0; }
+struct I8Part {
+    int s0, ns;  // 64-element steps s0 .. s0 + ns - 1
+    __host__ __device__ I8Part(int K, int rpg, int KS, int kp) {
+        if (i8_whole_groups(K, rpg)) {
+            const int G = K / 128, per = G / KS, rem = G % KS;
+            s0 = 2 * (kp * per + (kp < rem ? kp : rem));
+            ns = 2 * (per + (kp < rem));
+        } else {
+            const int steps = K / 64, spw = (steps + KS - 1) / KS;
+            s0 = kp * spw;
+            ns = spw < steps - s0 ? spw : steps - s0;
+        }
+    }
+};
+
 // Direct global->LDS copy of `pieces` 16-byte pieces (whole waves of them are
 // written: the LDS region is rounded up to 64 pieces).
 __device__ __forceinline__ void stage_block_issue(const uint4 *src, int pieces, uint4 *dst) {
@@ -82,7 +119,8 @@ __global__ __launch_bounds__(I8_MAX_KS *WAVE) void i8_gemv_kernel(const uint4 *W
     const int KS = blockDim.x / WAVE;
     const int tid = threadIdx.x, kp = __builtin_amdgcn_readfirstlane(tid / WAVE), lane = tid % WAVE, q = lane / 16,
               n = lane % 16;
-    const int steps = K / 64, spw = (steps + KS - 1) / KS, s0 = kp * spw, ns = min(spw, steps - s0);
+    const I8Part part(K, rpg, KS, kp);
+    const int steps = K / 64, s0 = part.s0, ns = part.ns;
     const int G = K / GRP, kc = x_row_stride(K);
     const int n0 = int(blockIdx.x) * 16;
     // activation slices of this tile: sl0 for its first row, sl1 for its last
@@ -153,7 +191,7 @@ __global__ __launch_bounds__(I8_MAX_KS *WAVE) void i8_gemv_kernel(const uint4 *W
                                 const int rows = mb == MB - 1 ? MR : 4;
 #pragma unroll
                                 for (int r = 0; r < 4; ++r)
-                                    if (r < rows) acc[j][mb][r] += sc[0] * ra[r] + sc[1] * rb[r];
+                                    if (r < rows) acc[j][mb][r] = i8_add32(acc[j][mb][r], sc[0], ra[r], sc[1], rb[r]);
                             }
                         }
                 } else {
@@ -167,13 +205,17 @@ __global__ __launch_bounds__(I8_MAX_KS *WAVE) void i8_gemv_kernel(const uint4 *W
                             for (int mb = 0; mb < MB; ++mb) {
                                 const uint2 *xh = reinterpret_cast<const uint2 *>(xr[j][mb]);
                                 const int rows = mb == MB - 1 ? MR : 4;
+                                f32x4 p;
 #pragma unroll
                                 for (int g = 0; g < 4; ++g) {
                                     const f32x4 rg = mfma16x16(xh[s * 16 + 4 * g + q], wg[g], zero);
 #pragma unroll
                                     for (int r = 0; r < 4; ++r)
-                                        if (r < rows) acc[j][mb][r] += sc[g] * rg[r];
+                                        if (r < rows) p[r] = g == 0 ? step_mul(sc[g], rg[r]) : __builtin_fmaf(sc[g], rg[r], p[r]);
                                 }
+#pragma unroll
+                                for (int r = 0; r < 4; ++r)
+                                    if (r < rows) acc[j][mb][r] = step_sum(acc[j][mb][r], p[r]);
                             }
                         }
                 }
@@ -230,7 +272,7 @@ __device__ __forceinline__ void i8_wide_block(const uint4 *Wt, const float *St, 
               q = lane / 16;
     const int item = int(blockIdx.x);
     const int nsub = (N + 15) / 16, steps = K / 64;
-    const int G = K / 128, per = G / WK, rem = G % WK;
+    const int G = K / 128, per = G / WK, rem = G % WK;  // (I8Part's split; parts past the last group are empty)
     const int g0 = wk * per + min(wk, rem), ng = per + (wk < rem), ngmax = per + (rem > 0);
     const uint4 *w[NS];
     const sv_t *sc[NS];
@@ -292,7 +334,9 @@ __device__ __forceinline__ void i8_wide_block(const uint4 *Wt, const float *St, 
 #pragma unroll
                     for (int mb = 0; mb < MB; ++mb) {
                         const f32x4 ra = mfma16<F16>(fa[mb], wa, zero), rb = mfma16<F16>(fb[mb], wb, zero);
-                        acc[j][mb] += r.s[j][t][0] * ra + r.s[j][t][1] * rb;
+#pragma unroll
+                        for (int e = 0; e < 4; ++e)
+                            acc[j][mb][e] = i8_add32(acc[j][mb][e], r.s[j][t][0], ra[e], r.s[j][t][1], rb[e]);
                     }
                 }
             } else {
@@ -305,9 +349,7 @@ __device__ __forceinline__ void i8_wide_block(const uint4 *Wt, const float *St, 
 #pragma unroll
                 for (int j = 0; j < NS; ++j) {
                     const uint32_t v[4] = {r.w[j][t].x, r.w[j][t].y, r.w[j][t].z, r.w[j][t].w};
-                    // the step's four groups first, so that the long sum has one
-                    // term per step as with groups of 32 (and 8 parts are no less
-                    // exact than the staged kernel's 16)
+                    const sv_t sj = r.s[j][t];
                     f32x4 p[MB];
 #pragma unroll
                     for (int g = 0; g < 4; ++g) {
@@ -315,11 +357,15 @@ __device__ __forceinline__ void i8_wide_block(const uint4 *Wt, const float *St, 
 #pragma unroll
                         for (int mb = 0; mb < MB; ++mb) {
                             const f32x4 rg = mfma16x16(f[mb][g], wg, zero);
-                            p[mb] = g == 0 ? r.s[j][t][g] * rg : p[mb] + r.s[j][t][g] * rg;
+#pragma unroll
+                            for (int e = 0; e < 4; ++e)
+                                p[mb][e] = g == 0 ? step_mul(sj[g], rg[e]) : __builtin_fmaf(sj[g], rg[e], p[mb][e]);
                         }
                     }
 #pragma unroll
-                    for (int mb = 0; mb < MB; ++mb) acc[j][mb] += p[mb];
+                    for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) acc[j][mb][e] = step_sum(acc[j][mb][e], p[mb][e]);
                 }
             }
         }
@@ -416,24 +462,30 @@ void launch_i8_tile(const int8_t *W8, const float *S, int N, int K, int group, u
     i8_tile_kernel<<<blocks, 256, 0, s>>>(W8, S, N, K, group, Wt, St);
 }
 
-// K split: up to 8 waves; 16 when the row tiles would not give every CU two
-// blocks (fewer blocks leave the weight stream short of loads in flight)
-static int i8_ks(int K, int N) {
+// Waves of the staged kernel: up to 8; 16 when the row tiles would not give
+// every CU two blocks (fewer blocks leave the weight stream short of loads in
+// flight). i8_ks_max: before the whole-group split (I8Part), which takes at most
+// 8 parts; the LDS limit is sized by it.
+static int i8_ks_max(int K, int N) {
     const int ks = (N + 15) / 16 < 512 ? 16 : 8;
     return K / 64 < ks ? K / 64 : ks;
+}
+static int i8_ks(int K, int N, int rpg) {
+    if (i8_whole_groups(K, rpg)) return K / 128 < 8 ? K / 128 : 8;
+    return i8_ks_max(K, N);
 }
 
 static int i8_nsl(int rpg) { return rpg > 0 && rpg % 16 != 0 ? 2 : 1; }
 
 size_t i8_lds_bytes(int M, int K, int N, int group, int rpg) {
-    const int KS = i8_ks(K, N), MB = M > 16 ? 2 : 1;
+    const int KS = i8_ks_max(K, N), MB = M > 16 ? 2 : 1;
     return size_t(x_pieces(i8_nsl(rpg) * M, K) + i8_scale_pieces(K, group)) * 16 +
            size_t(red_slots(KS, KS)) * MB * WAVE * 16;  // one set of k-split slots (no persistent blocks)
 }
 
 template <int GRP, int MB, int MR, int NSL>
 static void launch_i8_t(const I8Args &a, hipStream_t s) {
-    const int KS = i8_ks(a.K, a.N), threads = KS * WAVE;
+    const int KS = i8_ks(a.K, a.N, a.rpg), threads = KS * WAVE;
     const size_t lds = i8_lds_bytes(a.M, a.K, a.N, a.group, a.rpg);
     const int xpt = NSL == 1 ? (a.M * (a.K / 8) + threads - 1) / threads : 0;
     const unsigned blocks = unsigned((a.N + 15) / 16);
@@ -442,7 +494,7 @@ static void launch_i8_t(const I8Args &a, hipStream_t s) {
         kern<<<blocks, threads, lds, s>>>(a.W, a.S, a.x, a.xs, a.M, a.K, a.N, a.rpg, a.y, a.ys, a.y_bf16,
                                           a.accumulate);
     };
-    const int spw = (a.K / 64 + KS - 1) / KS;
+    const int spw = I8Part(a.K, a.rpg, KS, 0).ns;  // (the first part is the longest)
     auto pick = [&](auto ws) {
         constexpr int W = decltype(ws)::value;
         if constexpr (NSL == 2) go(i8_gemv_kernel<GRP, MB, MR, 0, W, 2>);

@@ -202,16 +202,31 @@ def test_gemv_ragged_k(gpu, oracle, N, K, M, f16):
     assert rel_err(host(y), oracle.q4_linear(W, S, Z, N, K, xf)) <= 1e-5  # fp32 sums of exact products
 
 
-# Rows streamed in K groups (batches of 9 to 32 whose rows do not fit LDS):
-# one and two 16-row blocks, a K split with unequal parts (43 groups) and
-# equal ones, 64- and 128- or 256-row blocks (N above 64 Ki rows), weight rows off
-# every block size.
-@pytest.mark.parametrize("N,K,M", [(1040, 6144, 12), (16, 11008, 16), (4112, 5504, 17), (528, 4096, 32), (3076 // 16 * 16, 3712, 25),
-                                   (65584, 6144, 9), (32848, 4096, 21)])
+def _staged_fits(M, K):
+    """Whether a batch's rows fit the staging LDS (gemv_fits, q4_gemv.hip): else 9 to 32 rows are streamed."""
+    G = K // 128
+    gpk = 4 * -(-G // 64)
+    ks = -(-G // gpk)
+    nw = next((w for w in (8, 12, 16) if w % ks == 0), 12 if 8 < ks <= 12 else 16)
+    waves = nw // ks * ks
+    stride = K // 8 | 1 if K // 8 >= 64 else K // 8
+    return -(-M * stride // 64) * 1024 + 2 * (waves - waves // ks) * (1 if M <= 16 else 2) * 1024 <= 160 * 1024
+
+
+# Rows streamed in K groups (batches of 9 to 32 whose rows do not fit LDS). Up to
+# 16 rows: 12 and 16 parts, parts longer than a chunk, a last part of 3 groups, and
+# chained blocks (N above 48 Ki) with an even and an odd number of parts. Above: the
+# 16-row blocks apart (N up to 8 Ki), together with one and with two parts per wave,
+# chained (N above 32 Ki). Weight rows off every block size.
+@pytest.mark.parametrize("N,K,M", [(1040, 6144, 12), (16, 11008, 16), (2064, 7040, 16), (65584, 6144, 13), (49232, 5504, 15),
+                                   (4112, 5504, 17), (528, 4096, 32), (3076 // 16 * 16, 3712, 25),
+                                   (8208, 3712, 32), (12304, 4096, 21), (8208, 6144, 32), (8224, 7040, 19),
+                                   (32848, 4096, 21), (32864, 2560, 32), (32784, 8320, 17)])
 @pytest.mark.parametrize("f16,zeros", [(False, True), (True, True), (False, False), (True, False)])
 def test_gemv_wide(gpu, oracle, N, K, M, f16, zeros):
     import torch
     print(f"gemv wide N={N} K={K} M={M} f16={f16} zeros={zeros}", flush=True)
+    assert M > 8 and not _staged_fits(M, K)
     g = torch.Generator(device=gpu)
     g.manual_seed(N + K)
     W = torch.randint(-2**31, 2**31, (N, K // 8), generator=g, device=gpu, dtype=torch.int32)
@@ -249,3 +264,33 @@ def test_gemv_wide_row_slices(gpu):
     for sl in (0, 5, ns - 1):
         whole = qwq4.gemv(*d, x[:, sl * K:(sl + 1) * K], N, K, M)
         assert torch.equal(y[:, sl * rpg:(sl + 1) * rpg], whole[:, sl * rpg:(sl + 1) * rpg])
+
+
+# Batches on both sides of every change of kernel (staged, streamed split and
+# chained): parts that cover K exactly and not, one and two parts per wave.
+@pytest.mark.parametrize("N,K,f16,zeros", [(1040, 4096, False, True), (4112, 6144, True, True), (4112, 6144, False, False),
+                                           (12304, 4096, True, False), (8208, 5504, False, True), (32848, 4096, False, True),
+                                           (32864, 2560, True, True), (49232, 7040, False, True), (1040, 8320, True, True)])
+def test_gemv_rows_independent_of_batch(gpu, N, K, f16, zeros):
+    """A token row's result is the same bits in every batch of 1 to 32 rows, infinities and NaN in
+    other rows and in its own included."""
+    import torch
+    print(f"gemv rows independent N={N} K={K} f16={f16} zeros={zeros}", flush=True)
+    assert not _staged_fits(32, K)
+    g = torch.Generator(device=gpu)
+    g.manual_seed(N + K)
+    W = torch.randint(-2**31, 2**31, (N, K // 8), generator=g, device=gpu, dtype=torch.int32)
+    S = (torch.randn((N, K // 128), generator=g, device=gpu) * 0.02).abs().to(torch.float16)
+    Z = torch.randint(-2**31, 2**31, (N, (K // 128 + 7) // 8), generator=g, device=gpu, dtype=torch.int32) if zeros else None
+    d = qwq4.tile(W, S, Z, N, K)
+    x = torch.randn((32, K), generator=g, device=gpu).to(torch.float16 if f16 else torch.bfloat16)
+    x[2, 130], x[20, K - 1], x[30, 0] = float("inf"), float("-inf"), float("nan")
+    y32 = qwq4.gemv(*d, x, N, K, 32)
+    ok = torch.ones(32, dtype=torch.bool, device=gpu)
+    ok[[2, 20, 30]] = False
+    assert bool(torch.isfinite(y32[ok]).all()) and not bool(torch.isfinite(y32[~ok]).any())
+    for M in (1, 2, 4, 8, 9, 11, 12, 16, 17, 20):
+        for m0 in {0, 32 - M}:
+            y, r = qwq4.gemv(*d, x[m0:m0 + M], N, K, M), y32[m0:m0 + M]
+            assert torch.equal(torch.isnan(y), torch.isnan(r)), (M, m0)
+            assert torch.equal(y.nan_to_num(nan=0.0).view(torch.int32), r.nan_to_num(nan=0.0).view(torch.int32)), (M, m0)

@@ -18,7 +18,7 @@ static void launch_gemv_fit(const GemvArgs &a, hipStream_t s) {
     else launch_gemv_fit_t<BF16>(a, s);
 }
 
-static void launch_gemv_rows(const GemvArgs &a, int n_all, hipStream_t s);
+static void launch_gemv_rows(const GemvArgs &a, hipStream_t s);
 
 // Rows grouped over activation slices (rpg > 0, the reference's
 // hyper-connection down projection: row n reads slice n / rpg of x, at
@@ -28,7 +28,7 @@ static void launch_gemv_rows(const GemvArgs &a, int n_all, hipStream_t s);
 // product of its own slice, with the same arithmetic as an ungrouped row.
 void launch_gemv(const GemvArgs &a, hipStream_t s) {
     if (a.rpg <= 0) {
-        launch_gemv_rows(a, a.N, s);
+        launch_gemv_rows(a, s);
         return;
     }
     const int G = a.K / QGROUP, GC = (G + 3) / 4;
@@ -44,23 +44,24 @@ void launch_gemv(const GemvArgs &a, hipStream_t s) {
         b.y = static_cast<char *>(a.y) + int64_t(b0) * ysz;
         b.N = r1 - b0;
         b.n_lo = r0 - b0;
-        launch_gemv_rows(b, a.N, s);
+        launch_gemv_rows(b, s);
     }
 }
 
-// Batches whose activations exceed LDS: from 9 rows on the streamed kernel
-// (one launch, the weights read once: 4096->12288 at 20 / 32 rows 17.0 / 18.8
-// -> 12.2 / 12.4 us, 6144->4096 at 12 / 32 11.5 / 20.0 -> 10.4 / 14.4; where
-// they do fit the staged kernel stays ahead, 2048->2048 at 20 rows 5.5 against
-// 7.1), below that several launches of fewer rows. (The streamed kernel
+// Batches whose activations exceed LDS: from 9 rows on the streamed kernel (one
+// launch, the weights read once: 4096->12288 at 20 / 32 rows 17.1 / 18.9 us in
+// several launches, 13.6 / 14.1 streamed, 6144->4096 13.5 / 20.2 and 12.0 / 12.3;
+// up to 16 rows of 6144 the two are about even; where the rows do fit the staged
+// kernel stays ahead, 4096->12288 at 16 rows 9.4 against 10.7), below that several
+// launches of fewer rows. All give a row the same bits. (The streamed kernel
 // addresses rows by 32-bit offsets.)
-static void launch_gemv_rows(const GemvArgs &a, int n_all, hipStream_t s) {
+static void launch_gemv_rows(const GemvArgs &a, hipStream_t s) {
     if (gemv_fits(a.M, a.K)) {
         launch_gemv_fit(a, s);
         return;
     }
     if (a.M > 8 && a.xs <= (1 << 25)) {
-        launch_gemv_wide(a, n_all, s);
+        launch_gemv_wide(a, s);
         return;
     }
     int mc = 16;

@@ -342,6 +342,11 @@ __device__ __forceinline__ void store_y(void *y, int64_t o, float v, int y_bf16,
 // partial sums: one slot per wave that is not a k-part 0, double-buffered
 __host__ __device__ inline int red_slots(int waves, int KS) { return waves - waves / KS; }
 
+// K split of the dense GEMV: parts of this many groups, the fewest whole chunks
+// that 16 waves cover G with (the last part shorter). A function of K alone: the
+// sums of every kernel and batch follow it.
+__host__ __device__ inline int dense_gpk(int G) { return 4 * ((G + 63) / 64); }
+
 // LDS: staged rows, then the partial-sum slots
 __host__ __device__ inline size_t dense_lds_bytes(int M, int K, int MB, int waves, int KS) {
     return size_t(x_pieces(M, K)) * 16 + size_t(2) * red_slots(waves, KS) * MB * WAVE * 16;

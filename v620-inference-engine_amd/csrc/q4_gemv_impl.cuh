@@ -37,9 +37,6 @@ namespace qwq4 {
 
 constexpr int DENSE_GW = 4;
 
-// K groups per wave: the fewest whole chunks that 16 waves cover G with.
-__host__ __device__ inline int dense_gpk(int G) { return 4 * ((G + 63) / 64); }
-
 template <typename XT, int NW, int MB, bool HAS_Z, bool PF, bool KSNW, int XPT, bool P4, int MR>
 // Argument order: what the weight and activation requests need first (the
 // first 14 dwords are preloaded into SGPRs at wave launch), the output last.

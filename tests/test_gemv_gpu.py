@@ -294,3 +294,20 @@ def test_gemv_rows_independent_of_batch(gpu, N, K, f16, zeros):
             y, r = qwq4.gemv(*d, x[m0:m0 + M], N, K, M), y32[m0:m0 + M]
             assert torch.equal(torch.isnan(y), torch.isnan(r)), (M, m0)
             assert torch.equal(y.nan_to_num(nan=0.0).view(torch.int32), r.nan_to_num(nan=0.0).view(torch.int32)), (M, m0)
+
+
+@pytest.mark.parametrize("G", [512, 530, 631])
+def test_gemv_longest_rows(gpu, oracle, G):
+    """K of 64 Ki, where a single row fits the staging LDS, and above, where none does beside the K parts'
+    sums: one row against the oracle, batches the same bits."""
+    import torch
+    N, K = 48, 128 * G
+    print(f"gemv longest rows K={K}", flush=True)
+    W, S, Z = synth.q4_weights(G, "long", N, K)
+    _, xf = synth.acts(G, "longx", 10, K)
+    d = qwq4.tile(to_dev(W, gpu), to_dev(S, gpu), to_dev(Z, gpu), N, K)
+    x = torch.from_numpy(xf).to(gpu).to(torch.bfloat16)
+    y = qwq4.gemv(*d, x[:1], N, K, 1)
+    assert rel_err(host(y), oracle.q4_linear_f64(W, S, Z, N, K, host(x[:1].float()))) <= 1e-5  # fp32 sums of exact products
+    for M in (2, 10):
+        assert torch.equal(qwq4.gemv(*d, x[:M], N, K, M)[:1], y)

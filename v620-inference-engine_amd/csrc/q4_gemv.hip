@@ -53,14 +53,15 @@ void launch_gemv(const GemvArgs &a, hipStream_t s) {
 // several launches, 13.6 / 14.1 streamed, 6144->4096 13.5 / 20.2 and 12.0 / 12.3;
 // up to 16 rows of 6144 the two are about even; where the rows do fit the staged
 // kernel stays ahead, 4096->12288 at 16 rows 9.4 against 10.7), below that several
-// launches of fewer rows. All give a row the same bits. (The streamed kernel
-// addresses rows by 32-bit offsets.)
+// launches of fewer rows; every batch is streamed where not even one row fits
+// beside the parts' sums (K above 65 Ki). All give a row the same bits. (The
+// streamed kernel addresses rows by 32-bit offsets.)
 static void launch_gemv_rows(const GemvArgs &a, hipStream_t s) {
     if (gemv_fits(a.M, a.K)) {
         launch_gemv_fit(a, s);
         return;
     }
-    if (a.M > 8 && a.xs <= (1 << 25)) {
+    if (a.M == 1 || (a.xs <= (1 << 25) && (a.M > 8 || !gemv_fits(1, a.K)))) {
         launch_gemv_wide(a, s);
         return;
     }
@@ -72,7 +73,7 @@ static void launch_gemv_rows(const GemvArgs &a, hipStream_t s) {
         b.M = a.M - m0 < mc ? a.M - m0 : mc;
         b.x = a.x + int64_t(m0) * a.xs;
         b.y = static_cast<char *>(a.y) + int64_t(m0) * a.ys * ysz;
-        launch_gemv_fit(b, s);
+        launch_gemv_rows(b, s);
     }
 }
 

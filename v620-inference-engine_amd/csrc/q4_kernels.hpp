@@ -33,7 +33,7 @@ struct GemvArgs {
     int n_lo = 0;   // rows below n_lo are computed but not stored (internal)
 };
 void launch_gemv(const GemvArgs &a, hipStream_t s);
-// 9 to 32 rows streamed through LDS in K groups (q4_gemv_wide.cuh).
+// 1 to 32 rows streamed through LDS in K groups (q4_gemv_wide.cuh).
 void launch_gemv_wide(const GemvArgs &a, hipStream_t s);
 
 // Weighted combine folded into the down projection (see launch_moe_gemv):

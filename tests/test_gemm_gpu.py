@@ -221,22 +221,50 @@ def test_gemm_saturation_and_nonfinite(gpu, oracle):
     assert np.all(~np.isfinite(Y[6]))
 
 
-# One shape per K-split tile (32 x 32, 32 x 64, 64 x 64, 64 x 128, 64 x 256,
-# 96 x 128, 96 x 256, 128 x 128, 128 x 256 tokens x weight rows) at sizes off
-# the tile edges, then the edges themselves: one weight subtile, one K group
-# (fewer than the block's parts), parts of unequal length (G = 13, 29), a
-# token over and under a tile.
+# The choice among the tiles of short chunks (SHAPES, q4_gemm_small.hip; 256 CUs):
+# tokens x weight rows and the fitted launch time.
+SMALL_TILES = [(32, 32, 2.231, 0.104, 0.148, 0.033, 1.011), (32, 64, 1.818, 0.046, 0.310, 0.064, 1.708),
+               (64, 64, 1.436, 0.0, 0.411, 0.102, 2.454), (96, 64, 0.084, 0.0, 0.529, 0.099, 4.245),
+               (128, 64, 0.0, 0.0, 0.595, 0.167, 4.296), (64, 128, 3.076, 0.370, 0.334, 0.217, 0.943),
+               (96, 128, 3.084, 0.302, 0.543, 0.218, 1.156), (128, 128, 5.737, 0.123, 0.806, 0.260, 0.207),
+               (128, 256, 0.0, 0.0, 1.642, 0.589, 5.009)]
+
+
+def _gemm_tile(T, N, K, cus=256):
+    """The tile a dense prefill GEMM takes: tokens x weight rows, (0, 0) for 256 x 256 tiles with
+    the rest as halves."""
+    def whole(nb):
+        return nb >= 4 * cus or nb >= cus and nb / cus - nb // cus < 0.01
+    t256 = -(-T // 256)
+    nb = -(-N // 256) * t256
+    if whole(nb):
+        return 256, 256
+    if nb > cus and 2 * (nb % cus) <= cus:
+        return 0, 0
+    if whole(-(-N // 128) * t256):
+        return 256, 128
+    blocks = [-(-N // bn) * -(-T // bm) for bm, bn, *_ in SMALL_TILES]
+    return min(zip(SMALL_TILES, blocks), key=lambda c: c[0][2] + K / 128 * (
+        c[0][3] + c[0][4] * -(-c[1] // cus) + c[0][5] * c[1] / cus) + c[0][6] * -(-c[1] // cus))[0][:2]
+
+
+# Every small tile at sizes off the tile edges, then the edges themselves: one
+# weight subtile, one K group, odd group counts (G = 13, 29), a token over and
+# under a tile.
 @pytest.mark.parametrize("T,N,K,zeros", [(21, 2048, 2048, True), (35, 5120, 2048, False), (43, 8704, 2048, True),
                                          (95, 12288, 2048, True), (1567, 5120, 1664, True), (502, 5120, 2048, False),
                                          (1074, 4096, 2048, True), (673, 4144, 3712, True), (1788, 8176, 1920, False),
                                          (1, 16, 128, True), (33, 48, 256, False), (32, 272, 1664, True),
-                                         (65, 2048, 3712, True), (129, 1040, 640, False)])
-def test_gemm_ksplit_shapes(gpu, oracle, T, N, K, zeros):
+                                         (65, 2048, 3712, True), (129, 1040, 640, False), (339, 5104, 2048, True),
+                                         (331, 8688, 384, False), (20, 8688, 128, True), (41, 8688, 128, False),
+                                         (300, 8688, 128, True), (970, 1040, 256, True), (1443, 1040, 256, False),
+                                         (970, 2064, 128, True), (601, 8688, 128, False), (3001, 8688, 128, True)])
+def test_gemm_small_tiles(gpu, oracle, T, N, K, zeros):
     """Strided fp16 rows and a strided output: fp32 rows within the tolerance
     of the oracle, nothing written past a row's N columns, and fp16 and bf16
     rows the roundings of the fp32 ones bit for bit."""
     import torch
-    print(f"gemm K-split T={T} N={N} K={K} zeros={zeros}", flush=True)
+    print(f"gemm small tiles T={T} N={N} K={K} zeros={zeros} tile={_gemm_tile(T, N, K)}", flush=True)
     W, S, Z = synth.q4_weights(T + N, f"ks{N}x{K}", N, K, zeros)
     _, xf = synth.acts(T + K, f"ksx{T}x{K}", T, K)
     x16 = xf.astype(np.float16)
@@ -259,7 +287,34 @@ def test_gemm_ksplit_shapes(gpu, oracle, T, N, K, zeros):
     assert rel_err(host(y32.contiguous())[np.ix_(toks, rows)], ref) <= TOL
 
 
-def test_gemm_ksplit_nonfinite(gpu, oracle):
+# Chunks on every kind of tile against one of 256 x 256 tiles (or those and halves)
+# that begins with the same rows; N off every tile edge, odd group counts.
+@pytest.mark.parametrize("N,K,T1,zeros,chunks", [
+    (4096, 1664, 4000, True, {47: (32, 32), 97: (32, 64), 200: (64, 64), 300: (96, 64), 449: (128, 64), 2340: (64, 128),
+                              600: (96, 128), 1000: (128, 128), 1600: (128, 256), 2000: (256, 128)}),
+    (4112, 896, 3969, False, {17: (32, 32), 65: (32, 64), 145: (64, 64), 241: (96, 64), 337: (128, 64), 900: (64, 128),
+                              460: (96, 128), 700: (128, 128), 1681: (128, 256)})])
+def test_gemm_rows_independent_of_chunk(gpu, N, K, T1, zeros, chunks):
+    """A token row's result is the same bits in a chunk of any length, infinities and NaN included."""
+    import torch
+    print(f"gemm rows independent N={N} K={K}", flush=True)
+    W, S, Z = synth.q4_weights(71, f"ri{N}x{K}", N, K, zeros)
+    dW, dS, dZ = qwq4.tile(to_dev(W, gpu), to_dev(S, gpu), to_dev(Z, gpu) if zeros else None, N, K)
+    g = torch.Generator(device=gpu)
+    g.manual_seed(N + K)
+    X = torch.randn((T1, K), generator=g, device=gpu).to(torch.float16)
+    X[3, K - 1], X[5, 64], X[11, 700] = float("inf"), float("-inf"), float("nan")
+    assert _gemm_tile(T1, N, K) in ((256, 256), (0, 0))
+    Y1 = qwq4.gemm(dW, dS, dZ, X, N, K, y_bf16=False).view(torch.int32)
+    nan = torch.isnan(Y1.view(torch.float32))
+    assert bool(nan[11].all()) and not bool(nan[12:].any())
+    for T, tile in chunks.items():
+        assert _gemm_tile(T, N, K) == tile, T
+        Y = qwq4.gemm(dW, dS, dZ, X[:T], N, K, y_bf16=False)
+        assert bool(((Y.view(torch.int32) == Y1[:T]) | (nan[:T] & torch.isnan(Y))).all()), (T, tile)
+
+
+def test_gemm_small_nonfinite(gpu, oracle):
     """Infinities and NaN in a row of a short chunk: what the plain product
     gives (an infinity times a zero weight is NaN, times any other an infinity
     of that sign), other rows untouched."""

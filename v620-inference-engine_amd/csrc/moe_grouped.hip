@@ -170,14 +170,6 @@ constexpr int LIGHT_A = 32 * 256;  // bytes of a group's A: [32][128] fp16
 // rows at one chunk of each 128-byte half
 __device__ __forceinline__ int light_swz(int r, int c) { return r * 256 + ((c ^ (r & 15)) << 4); }
 
-// dequant8's values, with one VALU instruction less: q - z exact, then the
-// rounding multiply. zl: -(1024 + z), zh: -(64 + z).
-__device__ __forceinline__ uint4 dequant8_light(uint32_t w, h2 zl, h2 zh, h2 s2) {
-    const uint4 d = unpack8_exact(w, zl, zh);
-    auto mul = [&](uint32_t v) { return __builtin_bit_cast(uint32_t, __builtin_bit_cast(h2, v) * s2); };
-    return make_uint4(mul(d.x), mul(d.y), mul(d.z), mul(d.w));
-}
-
 // acc[j] += the tile's 32 slots (A rows arow, this lane's of the loads) times
 // row group j's rows (b0, b1: row lane % 32) over all G groups; bs: the lane's
 // own row (its scales and zeros).

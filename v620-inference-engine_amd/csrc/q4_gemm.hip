@@ -13,7 +13,7 @@
 //
 // Schedule: q4_gemm_core.cuh (block tile 256 or 128 tokens x 256 weight
 // rows, 8 waves, LDS double-buffered K stages of 64), or for chunks with too
-// few such tiles the K-split tiles of q4_gemm_ksplit.cuh. Blocks take their tiles
+// few such tiles the small tiles of q4_gemm_small.cuh. Blocks take their tiles
 // in an XCD-aware order; the epilogue goes through LDS so that stores are
 // 16 bytes per lane.
 #include "q4_gemm_core.cuh"
@@ -130,11 +130,6 @@ static void launch_gemm_t(const GemmArgs &a, const uint16_t *Xh, int lda, hipStr
     kern<<<grid, G_THREADS, 0, s>>>(a.W, a.S, a.Z, Xh, lda, a.T, a.Y, a.ldy, a.N, a.K);
 }
 
-// 256 x 256 tiles when they fill whole rounds of the chip (or many rounds);
-// past one round with at most half a round left over, whole rounds of them
-// plus the rest as 256 x 128 halves in the same launch (2048-token
-// micro-batches of 4096->12288); else 256 tokens x 128 weight rows when those
-// fill whole rounds (the same dequant work per MFMA); else 128 x 256.
 template <bool HAS_Z, int YT>
 static void launch_gemm_mixed(const GemmArgs &a, const uint16_t *Xh, int lda, int nbig, int nhalf, hipStream_t s) {
     const int nbx = (a.N + 255) / 256;
@@ -142,17 +137,32 @@ static void launch_gemm_mixed(const GemmArgs &a, const uint16_t *Xh, int lda, in
         a.W, a.S, a.Z, Xh, lda, a.T, a.Y, a.ldy, a.N, a.K, nbx, nbig, nhalf);
 }
 
-template <bool HAS_Z, int YT>
-static void launch_gemm_m(const GemmArgs &a, const uint16_t *Xh, int lda, int cus, hipStream_t s) {
+enum class Tiles { T256, MIXED, T256x128, T128 };
+
+// 256 x 256 tiles when they fill whole rounds of the chip (or many rounds);
+// past one round with at most half a round left over, whole rounds of them
+// plus the rest as 256 x 128 halves in the same launch (2048-token
+// micro-batches of 4096->12288); else 256 tokens x 128 weight rows when those
+// fill whole rounds (the same dequant work per MFMA); else 128 x 256, or
+// the small tiles where they are faster.
+static Tiles pick_tiles(int N, int T, int cus) {
     auto whole = [&](int64_t nb) {
         const double rounds = double(nb) / cus;
         return rounds >= 4.0 || (rounds >= 1.0 && rounds - double(int64_t(rounds)) < 0.01);
     };
-    const int64_t t256 = (a.T + 255) / 256, nb = int64_t((a.N + 255) / 256) * t256;
-    if (whole(nb)) launch_gemm_t<HAS_Z, YT, 256>(a, Xh, lda, s);
-    else if (nb > cus && 2 * (nb % cus) <= cus)  // e.g. 2048 tokens x 12288 rows: 256 whole tiles + 256 halves
-        launch_gemm_mixed<HAS_Z, YT>(a, Xh, lda, int(nb / cus * cus), int(2 * (nb % cus)), s);
-    else if (whole(int64_t((a.N + 127) / 128) * t256)) launch_gemm_t<HAS_Z, YT, 256, 128>(a, Xh, lda, s);
+    const int64_t t256 = (int64_t(T) + 255) / 256, nb = (int64_t(N) + 255) / 256 * t256;
+    if (whole(nb)) return Tiles::T256;
+    if (nb > cus && 2 * (nb % cus) <= cus) return Tiles::MIXED;  // e.g. 2048 tokens x 12288 rows: 256 whole tiles + 256 halves
+    if (whole((int64_t(N) + 127) / 128 * t256)) return Tiles::T256x128;
+    return Tiles::T128;
+}
+
+template <bool HAS_Z, int YT>
+static void launch_gemm_m(const GemmArgs &a, const uint16_t *Xh, int lda, Tiles t, int cus, hipStream_t s) {
+    const int64_t nb = (int64_t(a.N) + 255) / 256 * ((int64_t(a.T) + 255) / 256);
+    if (t == Tiles::T256) launch_gemm_t<HAS_Z, YT, 256>(a, Xh, lda, s);
+    else if (t == Tiles::MIXED) launch_gemm_mixed<HAS_Z, YT>(a, Xh, lda, int(nb / cus * cus), int(2 * (nb % cus)), s);
+    else if (t == Tiles::T256x128) launch_gemm_t<HAS_Z, YT, 256, 128>(a, Xh, lda, s);
     else launch_gemm_t<HAS_Z, YT, 128>(a, Xh, lda, s);
 }
 
@@ -171,15 +181,16 @@ void launch_gemm(const GemmArgs &a, hipStream_t s) {
     (void)hipGetDevice(&dev);
     (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
     if (cus < 1) cus = 256;
-    if (launch_gemm_ksplit(a, Xh, lda, cus, s)) return;
+    const Tiles t = pick_tiles(a.N, a.T, cus);
+    if (t == Tiles::T128 && launch_gemm_small(a, Xh, lda, cus, s)) return;
     if (a.Z) {
-        if (a.y_type == 1) launch_gemm_m<true, 1>(a, Xh, lda, cus, s);
-        else if (a.y_type == 2) launch_gemm_m<true, 2>(a, Xh, lda, cus, s);
-        else launch_gemm_m<true, 0>(a, Xh, lda, cus, s);
+        if (a.y_type == 1) launch_gemm_m<true, 1>(a, Xh, lda, t, cus, s);
+        else if (a.y_type == 2) launch_gemm_m<true, 2>(a, Xh, lda, t, cus, s);
+        else launch_gemm_m<true, 0>(a, Xh, lda, t, cus, s);
     } else {
-        if (a.y_type == 1) launch_gemm_m<false, 1>(a, Xh, lda, cus, s);
-        else if (a.y_type == 2) launch_gemm_m<false, 2>(a, Xh, lda, cus, s);
-        else launch_gemm_m<false, 0>(a, Xh, lda, cus, s);
+        if (a.y_type == 1) launch_gemm_m<false, 1>(a, Xh, lda, t, cus, s);
+        else if (a.y_type == 2) launch_gemm_m<false, 2>(a, Xh, lda, t, cus, s);
+        else launch_gemm_m<false, 0>(a, Xh, lda, t, cus, s);
     }
 }
 

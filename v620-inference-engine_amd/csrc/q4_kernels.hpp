@@ -279,8 +279,8 @@ size_t gemm_workspace_bytes(int T, int K);
 // bf16 [T][ldx] -> fp16 [T][K] (saturating), the GEMMs' A operand.
 void launch_x_to_f16(const uint16_t *X, int ldx, int T, int K, uint16_t *Xh, hipStream_t s);
 void launch_gemm(const GemmArgs &a, hipStream_t s);
-// The K-split tiles on fp16 rows Xh (stride lda), where whole-K tiles would
-// leave CUs idle; false (nothing launched) elsewhere.
-bool launch_gemm_ksplit(const GemmArgs &a, const uint16_t *Xh, int lda, int cus, hipStream_t s);
+// The small tiles on fp16 rows Xh (stride lda), where 128 x 256 tiles would leave
+// CUs idle; false (nothing launched) where those are as fast.
+bool launch_gemm_small(const GemmArgs &a, const uint16_t *Xh, int lda, int cus, hipStream_t s);
 
 }  // namespace qwq4

@@ -839,27 +839,36 @@ static void launch_kind(const MoeGemvArgs &a, int max_active, int R, hipStream_t
     else launch_gate_up<KS, GW, HAS_Z, CH4>(a, max_active, R, s);
 }
 
+// The parts that occur (down_ks, pick_ks): the down projection's single part is
+// one group, its parts of 4 or 8 have 9 to 16 groups; gate/up has fewer than 4
+// parts only where they are an odd number of groups.
 template <bool DOWN, int KS, bool HAS_Z>
 static void launch_gw(const MoeGemvArgs &a, int max_active, int R, int gpk, hipStream_t s) {
-    // (a range shorter than GW requests its last group again: the down parts
-    // of F = 768 and 1152, 1280 have their own sizes)
-    if constexpr (DOWN) {
-        if (gpk == 3) {
-            launch_kind<DOWN, KS, 3, HAS_Z, false>(a, max_active, R, s);
-            return;
+    auto go = [&](auto gw, auto ch4) {
+        launch_kind<DOWN, KS, decltype(gw)::value, HAS_Z, decltype(ch4)::value>(a, max_active, R, s);
+    };
+    constexpr std::true_type ch4{};
+    constexpr std::false_type any{};
+    constexpr bool SHORT = !DOWN || KS <= 2, EVEN = DOWN ? KS > 1 : KS == 4;
+    if constexpr (SHORT) {
+        // (a range shorter than GW requests its last group again: the down parts
+        // of F = 768 and 1152, 1280 have their own sizes)
+        if constexpr (DOWN && KS == 2) {
+            if (gpk == 3) return go(std::integral_constant<int, 3>(), any);
+            if (gpk == 5) return go(std::integral_constant<int, 5>(), any);
         }
-        if (gpk == 5) {
-            launch_kind<DOWN, KS, 5, HAS_Z, false>(a, max_active, R, s);
-            return;
+        if constexpr (EVEN) {
+            if (gpk == 4) return go(std::integral_constant<int, 4>(), ch4);
+            if (gpk == 6) return go(std::integral_constant<int, 6>(), any);  // down at F = 1536 (1408: 6 + 5)
+            if (gpk == 8) return go(std::integral_constant<int, 8>(), ch4);
         }
+        if (gpk < 4 || (DOWN && KS == 1)) return go(std::integral_constant<int, 4>(), any);
+        if constexpr (!(DOWN && KS == 1))
+            if (gpk < 8) return go(std::integral_constant<int, 8>(), any);
     }
-    if (gpk == 4) launch_kind<DOWN, KS, 4, HAS_Z, true>(a, max_active, R, s);
-    else if (gpk < 4) launch_kind<DOWN, KS, 4, HAS_Z, false>(a, max_active, R, s);
-    else if (gpk == 6) launch_kind<DOWN, KS, 6, HAS_Z, false>(a, max_active, R, s);  // down at F = 1536 (1408: 6 + 5)
-    else if (gpk == 8) launch_kind<DOWN, KS, 8, HAS_Z, true>(a, max_active, R, s);
-    else if (gpk < 8) launch_kind<DOWN, KS, 8, HAS_Z, false>(a, max_active, R, s);
-    else if (gpk % 4 == 0) launch_kind<DOWN, KS, 16, HAS_Z, true>(a, max_active, R, s);
-    else launch_kind<DOWN, KS, 16, HAS_Z, false>(a, max_active, R, s);
+    if constexpr (EVEN)
+        if (gpk % 4 == 0) return go(std::integral_constant<int, 16>(), ch4);
+    if constexpr (!(DOWN && KS == 1)) go(std::integral_constant<int, 16>(), any);
 }
 
 template <bool DOWN, bool HAS_Z>

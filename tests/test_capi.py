@@ -114,3 +114,17 @@ def test_workspace_sizes():
     assert qwq4.lib().qw_w16_tiled_size(3073, 4096) == 3088 * 4096 * 2
     assert qwq4.gemm_workspace_size(4096, 4096) >= 4096 * 4096 * 2
     assert qwq4.lib().qw_q4_gemm_workspace_size(0, 4096) == 0
+
+
+def test_stream_handle(monkeypatch):
+    """The binding's stream is the current device's current one, by torch's raw handle or, where
+    torch has none, by the Stream object's."""
+    import types
+
+    import torch
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: 1)
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda d=None: types.SimpleNamespace(cuda_stream=70 + d))
+    monkeypatch.setattr(torch._C, "_cuda_getCurrentRawStream", lambda d: 90 + d, raising=False)
+    assert qwq4._stream() == 91
+    monkeypatch.delattr(torch._C, "_cuda_getCurrentRawStream")
+    assert qwq4._stream() == 71

@@ -375,7 +375,8 @@ def test_grouped_light_loads(gpu, oracle, E, H, F, zeros, yp16):
 @pytest.mark.parametrize("E,H,F,zeros,yp16", [(64, 640, 384, True, True), (64, 1152, 640, False, False)])
 def test_grouped_rows_independent(gpu, E, H, F, zeros, yp16):
     """A token's expert rows do not depend on the length of its chunk: h, the
-    experts' outputs and the combined rows equal, bit for bit."""
+    experts' outputs and the combined rows equal, bit for bit, rows with
+    infinities and NaN included."""
     import torch
     k, T0, T1 = 4, 90, 1500
     print(f"grouped rows E={E} H={H} F={F} zeros={zeros}", flush=True)
@@ -383,6 +384,7 @@ def test_grouped_rows_independent(gpu, E, H, F, zeros, yp16):
     l[:40, 11] += 8.0  # one expert of over 32 of the short chunk's tokens
     ex = synth.experts(64, E, H, F, zeros=zeros)
     xb, _ = synth.acts(64, f"li{H}", T1, H)
+    xb[3, H - 1], xb[17, 200], xb[41, 0] = 0x7F80, 0xFF80, 0x7FC0  # bf16 infinities and NaN
     from test_moe_gpu import _experts_dev
     (dg, du, dd), E, F = _experts_dev(gpu, ex)
     assert _light_load(T0, k, E, H, F) and not _light_load(T1, k, E, H, F)
@@ -392,5 +394,7 @@ def test_grouped_rows_independent(gpu, E, H, F, zeros, yp16):
         h, yp = qwq4.moe_experts_grouped(dg, du, dd, r, to_dev(xb[:T], gpu), E, F, yp_f16=yp16)
         slots = r.tok_slot[:T0].long()
         got.append([h[slots], yp[slots], qwq4.moe_combine(yp, r, H, out_bf16=False)[:T0]])
+    ok = [t for t in range(T0) if t not in (3, 17, 41)]
     for a, b in zip(*got):
-        assert torch.equal(a, b)
+        assert bool(torch.isfinite(a[ok].float()).all()) and not bool(torch.isfinite(a[3].float()).all())
+        assert bool(((a == b) | (torch.isnan(a) & torch.isnan(b))).all())

@@ -70,17 +70,17 @@ def test_i8_gemv_grouped_rows(gpu, oracle, group, M):
         assert rel_err(y, oracle.i8_linear_f64(W8, S, x16, M, xs=HC * SH, rpg=rpg, group=group)) <= TOL
 
 
-@pytest.mark.parametrize("group", [32, 16])
-@pytest.mark.parametrize("N,K,M", [(16, 128, 1), (20, 384, 9), (4097, 1152, 4), (8200, 256, 15), (8200, 1152, 17),
-                                   (8193, 128, 5), (12289, 640, 16), (12300, 1152, 32), (16400, 2176, 29),
-                                   (300, 192, 11)])
-def test_i8_gemv_streamed(gpu, group, N, K, M):
-    """The streamed kernel's shapes (1 to 4 row tiles per block, one and two row blocks,
-    K parts of unequal and zero groups, ragged rows and tiles), fp16 rows between wider
-    ones, fp32 and bf16 results and accumulation. Integer activations and power-of-two
-    scales: partial sums are exact fp32 integers times 2^-3, so results are bit-exact."""
+def _streamed(N, K, M, group):
+    """Which kernel an ungrouped call takes (i8_wide, i8_gemv.hip)."""
+    nt = -(-N // 16)
+    return K % 128 == 0 and (M > 8 or nt <= 768 and not (group == 16 and M == 1 and nt > 640))
+
+
+def _check_exact(gpu, group, N, K, M):
+    """fp16 rows between wider ones, fp32 and bf16 results and accumulation. Integer
+    activations and power-of-two scales: partial sums are exact fp32 integers times
+    2^-3, so results are bit-exact."""
     import torch
-    print(f"i8 gemv streamed group={group} N={N} K={K} M={M}", flush=True)
     rng = np.random.default_rng(N + K + M)
     W8 = rng.integers(-128, 128, size=(N, K), dtype=np.int8)
     S = np.ldexp(1.0, rng.integers(-3, 2, size=(N, K // group))).astype(np.float32)
@@ -97,6 +97,31 @@ def test_i8_gemv_streamed(gpu, group, N, K, M):
     assert np.array_equal(yh[:, :N], (ref + 2.0).astype(np.float32))
     yb = host(qwq4.gemv_i8(Wt, St, N, K, xd, M, group=group, xs=K + 8, y_bf16=True))
     assert bf16_err_ok(yb, ref)
+
+
+@pytest.mark.parametrize("group", [32, 16])
+@pytest.mark.parametrize("N,K,M", [(16, 128, 1), (20, 384, 9), (4097, 1152, 4), (8200, 256, 15), (8200, 1152, 17),
+                                   (8193, 128, 5), (12289, 640, 16), (12300, 1152, 32), (16400, 2176, 29)])
+def test_i8_gemv_streamed(gpu, group, N, K, M):
+    """One to four row tiles per block, one and two row blocks, K parts of unequal and zero
+    groups, ragged rows and tiles."""
+    print(f"i8 gemv streamed group={group} N={N} K={K} M={M}", flush=True)
+    assert _streamed(N, K, M, group)
+    _check_exact(gpu, group, N, K, M)
+
+
+# Rows staged whole: up to 8 rows of more than 768 tiles (through registers and by
+# direct loads, short and long K ranges per wave), one row with groups of 16 of 641
+# to 768 tiles, and K an odd multiple of 64 at any batch (one and two row blocks, and
+# rows that take several launches).
+@pytest.mark.parametrize("group,N,K,M", [(g, n, k, m) for g in (32, 16) for n, k, m in (
+    (12304, 2048, 1), (12304, 2048, 2), (12290, 2048, 8), (12304, 6144, 3), (12290, 6144, 1), (12290, 6144, 8),
+    (12304, 128, 4), (12304, 1152, 5), (1000, 4160, 8), (520, 4160, 17), (8200, 4160, 32), (270, 4160, 9),
+    (12304, 1088, 16), (300, 192, 11))] + [(16, 12288, 4096, 1), (16, 10250, 1664, 1)])
+def test_i8_gemv_staged(gpu, group, N, K, M):
+    print(f"i8 gemv staged group={group} N={N} K={K} M={M}", flush=True)
+    assert not _streamed(N, K, M, group)
+    _check_exact(gpu, group, N, K, M)
 
 
 def test_i8_gemv_rows_independent(gpu, oracle):
@@ -117,9 +142,10 @@ def test_i8_gemv_rows_independent(gpu, oracle):
 # than parts.
 @pytest.mark.parametrize("group", [32, 16])
 @pytest.mark.parametrize("N,K", [(12304, 2048), (12289, 1152), (12300, 384), (12288, 1664), (10256, 4096), (4096, 6144),
-                                 (1000, 896), (300, 192)])
+                                 (1000, 896), (300, 192), (520, 4160)])
 def test_i8_gemv_rows_independent_of_batch(gpu, group, N, K):
-    """A token row's result is the same bits in every batch of 1 to 32 rows."""
+    """A token row's result is the same bits in every batch of 1 to 32 rows, infinities and NaN in
+    other rows and in its own included."""
     import torch
     print(f"i8 rows independent group={group} N={N} K={K}", flush=True)
     g = torch.Generator(device=gpu)
@@ -127,12 +153,17 @@ def test_i8_gemv_rows_independent_of_batch(gpu, group, N, K):
     W8 = torch.randint(-127, 128, (N, K), generator=g, device=gpu, dtype=torch.int32).to(torch.int8)
     S = (torch.randn((N, K // group), generator=g, device=gpu) * 0.002).abs()
     x = torch.randn((32, K), generator=g, device=gpu).to(torch.float16)
+    x[2, 130], x[20, K - 1], x[30, 0] = float("inf"), float("-inf"), float("nan")
     Wt, St = qwq4.i8_tile(W8, S, group)
     y32 = qwq4.gemv_i8(Wt, St, N, K, x, 32, group=group)
+    ok = torch.ones(32, dtype=torch.bool, device=gpu)
+    ok[[2, 20, 30]] = False
+    assert bool(torch.isfinite(y32[ok]).all()) and not bool(torch.isfinite(y32[~ok]).any())
     for M in (1, 2, 3, 8, 9, 16, 17):
         for m0 in {0, 32 - M}:
-            y = qwq4.gemv_i8(Wt, St, N, K, x[m0:m0 + M], M, group=group)
-            assert torch.equal(y.view(torch.int32), y32[m0:m0 + M].view(torch.int32)), (M, m0)
+            y, r = qwq4.gemv_i8(Wt, St, N, K, x[m0:m0 + M], M, group=group), y32[m0:m0 + M]
+            assert torch.equal(torch.isnan(y), torch.isnan(r)), (M, m0)
+            assert torch.equal(y.nan_to_num(nan=0.0).view(torch.int32), r.nan_to_num(nan=0.0).view(torch.int32)), (M, m0)
 
 
 def test_i8_gemv_strides_bf16_out_and_accumulate(gpu, oracle):

@@ -580,7 +580,8 @@ static int pick_ks(int G, int kmax) {
 // Down projection: a split of 2 where a wave's range stays within 16 groups
 // (fewer, larger blocks: each has more weight bytes in flight for its fixed
 // costs), else up to 8; the last part takes what is left. (Equal parts left odd
-// group counts unsplit, 128 rows per block: DOWN_ODD_F.)
+// group counts unsplit, 128 rows per block: four blocks of 256 experts, F = 1408
+// at batch 1 128 against 108 us, F = 1152 at batch 11 307 against 271.)
 static int down_ks(int G) {
     int ks = G > 1 ? 2 : 1;
     while ((G + ks - 1) / ks > 16 && ks < 8) ks *= 2;

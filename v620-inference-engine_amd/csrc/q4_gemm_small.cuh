@@ -9,8 +9,9 @@
 // Roles form (up to a few hundred tokens): NP waves move A (direct global -> LDS
 // loads) and dequantise the block's weight rows into LDS, a group (128 K) ahead;
 // the others hold 32 NI x 32 NJ results each and only read fragments and run
-// MFMAs. Bound by the chain of MFMAs over K, about 650 cycles a group with its
-// fragment reads and barrier (6144->4096 at 16 tokens 16 us). With loads,
+// MFMAs. Bound by the latency of a group's turn (8 MFMAs in a chain, fragment
+// reads, barrier): about 650 cycles for 32 x 32 (6144->4096 at 16 tokens 16 us),
+// which neither twice the loading waves nor two fragment sets shorten. With loads,
 // dequantisation and MFMAs in the same waves it was the sum of them (22 us).
 //
 // Register form (beyond that): a wave holds 32 weight rows and every token row of

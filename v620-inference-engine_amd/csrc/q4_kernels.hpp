@@ -151,7 +151,7 @@ struct RouterArgs {
 // Up to 8 tokens: the shared expert's gate/up GEMV in the router-logits launch
 // (and at batch 1 its down GEMV beside the routed gate/up) where the shapes
 // allow (T <= 8, H a multiple of 256 up to 8192, Fs of 32 from 256 to 4096: the
-// 16-bit GEMVs then run their 8 waves, the last with fewer steps).
+// 16-bit GEMVs then run their 8 waves, the last ones with fewer steps or none).
 bool shared_logits_ok(int T, int H, int Fs);
 void launch_router_logits_shgu(const RouterArgs &r, int T, int E, const ShExpertArgs &sh, hipStream_t s);
 // 2 to 4 tokens: the routing (one block, as launch_route) and the shared

@@ -221,31 +221,37 @@ def test_gemm_saturation_and_nonfinite(gpu, oracle):
     assert np.all(~np.isfinite(Y[6]))
 
 
-# The choice among the tiles of short chunks (SHAPES, q4_gemm_small.hip; 256 CUs):
-# tokens x weight rows and the fitted launch time.
-SMALL_TILES = [(32, 32, 2.231, 0.104, 0.148, 0.033, 1.011), (32, 64, 1.818, 0.046, 0.310, 0.064, 1.708),
-               (64, 64, 1.436, 0.0, 0.411, 0.102, 2.454), (96, 64, 0.084, 0.0, 0.529, 0.099, 4.245),
-               (128, 64, 0.0, 0.0, 0.595, 0.167, 4.296), (64, 128, 3.076, 0.370, 0.334, 0.217, 0.943),
-               (96, 128, 3.084, 0.302, 0.543, 0.218, 1.156), (128, 128, 5.737, 0.123, 0.806, 0.260, 0.207),
-               (128, 256, 0.0, 0.0, 1.642, 0.589, 5.009)]
+# The choice of the dense prefill GEMM's tile (pick_tiles, q4_gemm.hip; SHAPES,
+# q4_gemm_small.hip; 256 CUs): tokens x weight rows and the fitted launch time.
+SMALL_TILES = [(32, 32, 1.244, 0.110, 0.139, 0.038, 1.931), (32, 64, 1.185, 0.044, 0.311, 0.066, 2.353),
+               (64, 64, 0.823, 0.029, 0.383, 0.103, 3.072), (96, 64, 0.480, 0.0, 0.555, 0.064, 3.823),
+               (128, 64, 0.202, 0.0, 0.620, 0.136, 3.879), (64, 128, 3.008, 0.307, 0.330, 0.274, 1.020),
+               (96, 128, 2.171, 0.265, 0.498, 0.320, 1.453), (128, 128, 2.871, 0.144, 0.750, 0.325, 1.985)]
 
 
 def _gemm_tile(T, N, K, cus=256):
-    """The tile a dense prefill GEMM takes: tokens x weight rows, (0, 0) for 256 x 256 tiles with
-    the rest as halves."""
+    """Its tokens x weight rows, (0, 0) for 256 x 256 tiles with the rest as halves."""
     def whole(nb):
         return nb >= 4 * cus or nb >= cus and nb / cus - nb // cus < 0.01
-    t256 = -(-T // 256)
-    nb = -(-N // 256) * t256
+
+    def blocks(bm, bn):
+        return -(-N // bn) * -(-T // bm)
+
+    def us(nb, rounds, base, per_k, per_round, per_load, per_launch_round):
+        return base + K / 128 * (per_k + per_round * rounds + per_load * nb / cus) + per_launch_round * rounds
+    nb = blocks(256, 256)
     if whole(nb):
-        return 256, 256
-    if nb > cus and 2 * (nb % cus) <= cus:
-        return 0, 0
-    if whole(-(-N // 128) * t256):
-        return 256, 128
-    blocks = [-(-N // bn) * -(-T // bm) for bm, bn, *_ in SMALL_TILES]
-    return min(zip(SMALL_TILES, blocks), key=lambda c: c[0][2] + K / 128 * (
-        c[0][3] + c[0][4] * -(-c[1] // cus) + c[0][5] * c[1] / cus) + c[0][6] * -(-c[1] // cus))[0][:2]
+        large = us(nb, -(-nb // cus), 0.0, 0.238, 1.820, 1.695, 8.705), (256, 256)
+    elif nb > cus and 2 * (nb % cus) <= cus:
+        large = us(nb, nb // cus + 0.5, 0.0, 0.301, 2.069, 1.625, 6.589), (0, 0)
+    elif whole(blocks(256, 128)):
+        nb = blocks(256, 128)
+        large = us(nb, -(-nb // cus), 0.0, 0.007, 1.166, 0.878, 5.586), (256, 128)
+    else:
+        nb = blocks(128, 256)
+        large = us(nb, -(-nb // cus), 0.024, 0.023, 1.506, 0.718, 5.149), (128, 256)
+    small = [(us(blocks(bm, bn), -(-blocks(bm, bn) // cus), *t), (bm, bn)) for bm, bn, *t in SMALL_TILES]
+    return min([large] + small)[1]
 
 
 # Every small tile at sizes off the tile edges, then the edges themselves: one
@@ -257,8 +263,9 @@ def _gemm_tile(T, N, K, cus=256):
                                          (1, 16, 128, True), (33, 48, 256, False), (32, 272, 1664, True),
                                          (65, 2048, 3712, True), (129, 1040, 640, False), (339, 5104, 2048, True),
                                          (331, 8688, 384, False), (20, 8688, 128, True), (41, 8688, 128, False),
-                                         (300, 8688, 128, True), (970, 1040, 256, True), (1443, 1040, 256, False),
-                                         (970, 2064, 128, True), (601, 8688, 128, False), (3001, 8688, 128, True)])
+                                         (300, 8688, 128, True), (970, 1040, 256, True), (1750, 1040, 256, False),
+                                         (290, 4096, 1664, True), (601, 8688, 128, False), (3001, 8688, 128, True),
+                                         (5, 33040, 256, True), (63, 66064, 128, False), (390, 4112, 896, True)])
 def test_gemm_small_tiles(gpu, oracle, T, N, K, zeros):
     """Strided fp16 rows and a strided output: fp32 rows within the tolerance
     of the oracle, nothing written past a row's N columns, and fp16 and bf16
@@ -290,10 +297,11 @@ def test_gemm_small_tiles(gpu, oracle, T, N, K, zeros):
 # Chunks on every kind of tile against one of 256 x 256 tiles (or those and halves)
 # that begins with the same rows; N off every tile edge, odd group counts.
 @pytest.mark.parametrize("N,K,T1,zeros,chunks", [
-    (4096, 1664, 4000, True, {47: (32, 32), 97: (32, 64), 200: (64, 64), 300: (96, 64), 449: (128, 64), 2340: (64, 128),
+    (4096, 1664, 4000, True, {47: (32, 32), 97: (32, 64), 200: (64, 64), 300: (96, 64), 449: (128, 64),
                               600: (96, 128), 1000: (128, 128), 1600: (128, 256), 2000: (256, 128)}),
-    (4112, 896, 3969, False, {17: (32, 32), 65: (32, 64), 145: (64, 64), 241: (96, 64), 337: (128, 64), 900: (64, 128),
-                              460: (96, 128), 700: (128, 128), 1681: (128, 256)})])
+    (4112, 896, 4065, False, {17: (32, 32), 65: (32, 64), 145: (64, 64), 241: (96, 64), 337: (128, 64), 400: (64, 128),
+                              460: (96, 128), 700: (128, 128), 1681: (128, 256)}),
+    (33040, 256, 450, True, {5: (64, 128), 100: (128, 256)})])
 def test_gemm_rows_independent_of_chunk(gpu, N, K, T1, zeros, chunks):
     """A token row's result is the same bits in a chunk of any length, infinities and NaN included."""
     import torch
@@ -303,7 +311,7 @@ def test_gemm_rows_independent_of_chunk(gpu, N, K, T1, zeros, chunks):
     g = torch.Generator(device=gpu)
     g.manual_seed(N + K)
     X = torch.randn((T1, K), generator=g, device=gpu).to(torch.float16)
-    X[3, K - 1], X[5, 64], X[11, 700] = float("inf"), float("-inf"), float("nan")
+    X[3, K - 1], X[5, 64], X[11, K // 2] = float("inf"), float("-inf"), float("nan")
     assert _gemm_tile(T1, N, K) in ((256, 256), (0, 0))
     Y1 = qwq4.gemm(dW, dS, dZ, X, N, K, y_bf16=False).view(torch.int32)
     nan = torch.isnan(Y1.view(torch.float32))

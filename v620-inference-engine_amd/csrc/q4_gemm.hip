@@ -143,17 +143,35 @@ enum class Tiles { T256, MIXED, T256x128, T128 };
 // past one round with at most half a round left over, whole rounds of them
 // plus the rest as 256 x 128 halves in the same launch (2048-token
 // micro-batches of 4096->12288); else 256 tokens x 128 weight rows when those
-// fill whole rounds (the same dequant work per MFMA); else 128 x 256, or
-// the small tiles where they are faster.
-static Tiles pick_tiles(int N, int T, int cus) {
+// fill whole rounds (the same dequant work per MFMA); else 128 x 256. us: the
+// launch's predicted time; where a small tile takes less that one runs (chunks
+// that leave CUs idle, or wide matrices with few tokens, whose 256-token tiles
+// are padding: 65536 rows of K = 4096 at 1 / 80 tokens 124 / 119 us against 53 /
+// 63, 151936 rows at 40 tokens 304 against 110).
+static Tiles pick_tiles(int N, int K, int T, int cus, float &us) {
     auto whole = [&](int64_t nb) {
         const double rounds = double(nb) / cus;
         return rounds >= 4.0 || (rounds >= 1.0 && rounds - double(int64_t(rounds)) < 0.01);
     };
-    const int64_t t256 = (int64_t(T) + 255) / 256, nb = (int64_t(N) + 255) / 256 * t256;
-    if (whole(nb)) return Tiles::T256;
-    if (nb > cus && 2 * (nb % cus) <= cus) return Tiles::MIXED;  // e.g. 2048 tokens x 12288 rows: 256 whole tiles + 256 halves
-    if (whole((int64_t(N) + 127) / 128 * t256)) return Tiles::T256x128;
+    auto blocks = [&](int bm, int bn) { return (int64_t(N) + bn - 1) / bn * ((int64_t(T) + bm - 1) / bm); };
+    auto time = [&](TileTime t, int64_t nb, float rounds) { return t.us(K / QGROUP, float(nb) / float(cus), rounds); };
+    auto ceil_rounds = [&](int64_t nb) { return float((nb + cus - 1) / cus); };
+    int64_t nb = blocks(256, 256);
+    if (whole(nb)) {
+        us = time({0.f, 0.238f, 1.820f, 1.695f, 8.705f}, nb, ceil_rounds(nb));
+        return Tiles::T256;
+    }
+    if (nb > cus && 2 * (nb % cus) <= cus) {  // e.g. 2048 tokens x 12288 rows: 256 whole tiles + 256 halves
+        us = time({0.f, 0.301f, 2.069f, 1.625f, 6.589f}, nb, float(nb / cus) + 0.5f);
+        return Tiles::MIXED;
+    }
+    nb = blocks(256, 128);
+    if (whole(nb)) {
+        us = time({0.f, 0.007f, 1.166f, 0.878f, 5.586f}, nb, ceil_rounds(nb));
+        return Tiles::T256x128;
+    }
+    nb = blocks(128, 256);
+    us = time({0.024f, 0.023f, 1.506f, 0.718f, 5.149f}, nb, ceil_rounds(nb));
     return Tiles::T128;
 }
 
@@ -181,8 +199,9 @@ void launch_gemm(const GemmArgs &a, hipStream_t s) {
     (void)hipGetDevice(&dev);
     (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
     if (cus < 1) cus = 256;
-    const Tiles t = pick_tiles(a.N, a.T, cus);
-    if (t == Tiles::T128 && launch_gemm_small(a, Xh, lda, cus, s)) return;
+    float us;
+    const Tiles t = pick_tiles(a.N, a.K, a.T, cus, us);
+    if (launch_gemm_small(a, Xh, lda, cus, us, s)) return;
     if (a.Z) {
         if (a.y_type == 1) launch_gemm_m<true, 1>(a, Xh, lda, t, cus, s);
         else if (a.y_type == 2) launch_gemm_m<true, 2>(a, Xh, lda, t, cus, s);

@@ -7,22 +7,15 @@ namespace qwq4 {
 
 namespace {
 
-// A tile of bm tokens x bn weight rows and its launch time in us over nb blocks
-// and G groups of 128 K: base + G (per_k + per_round R + per_load nb / CUs) + round R,
-// with R rounds of one block per CU. Fitted to 138 launches of seeded random shapes
-// (N 512-14336, K 1024-8192, 1-3900 tokens): the tile predicted fastest is within
-// 0.3% of the one measured fastest on average, at worst 13% (4672 rows of K = 7040,
-// 435 tokens). The last is the 128 x 256 whole-chip tile (q4_gemm.hip).
-struct Shape {
+struct Shape {  // a tile of bm tokens x bn weight rows
     int bm, bn;
-    float base, per_k, per_round, per_load, round;
+    TileTime t;
 };
 constexpr Shape SHAPES[] = {
-    {32, 32, 2.231f, 0.104f, 0.148f, 0.033f, 1.011f}, {32, 64, 1.818f, 0.046f, 0.310f, 0.064f, 1.708f},
-    {64, 64, 1.436f, 0.f, 0.411f, 0.102f, 2.454f},    {96, 64, 0.084f, 0.f, 0.529f, 0.099f, 4.245f},
-    {128, 64, 0.f, 0.f, 0.595f, 0.167f, 4.296f},      {64, 128, 3.076f, 0.370f, 0.334f, 0.217f, 0.943f},
-    {96, 128, 3.084f, 0.302f, 0.543f, 0.218f, 1.156f}, {128, 128, 5.737f, 0.123f, 0.806f, 0.260f, 0.207f},
-    {128, 256, 0.f, 0.f, 1.642f, 0.589f, 5.009f},
+    {32, 32, {1.244f, 0.110f, 0.139f, 0.038f, 1.931f}},  {32, 64, {1.185f, 0.044f, 0.311f, 0.066f, 2.353f}},
+    {64, 64, {0.823f, 0.029f, 0.383f, 0.103f, 3.072f}},  {96, 64, {0.480f, 0.f, 0.555f, 0.064f, 3.823f}},
+    {128, 64, {0.202f, 0.f, 0.620f, 0.136f, 3.879f}},    {64, 128, {3.008f, 0.307f, 0.330f, 0.274f, 1.020f}},
+    {96, 128, {2.171f, 0.265f, 0.498f, 0.320f, 1.453f}}, {128, 128, {2.871f, 0.144f, 0.750f, 0.325f, 1.985f}},
 };
 
 template <class Kern>
@@ -46,19 +39,16 @@ void launch_roles(const GemmArgs &a, const uint16_t *Xh, int lda, hipStream_t s)
 
 }  // namespace
 
-bool launch_gemm_small(const GemmArgs &a, const uint16_t *Xh, int lda, int cus, hipStream_t s) {
+bool launch_gemm_small(const GemmArgs &a, const uint16_t *Xh, int lda, int cus, float large_us, hipStream_t s) {
     if (lda > (1 << 23)) return false;  // (token rows within a tile are addressed by 32-bit offsets)
-    int best = 0;
-    float t = 0.f;
-    const float G = float(a.K / QGROUP);
+    int best = -1;
     for (int i = 0; i < int(sizeof SHAPES / sizeof SHAPES[0]); ++i) {
         const Shape &p = SHAPES[i];
         const int64_t nb = (int64_t(a.N) + p.bn - 1) / p.bn * ((int64_t(a.T) + p.bm - 1) / p.bm);
-        const float R = float((nb + cus - 1) / cus);
-        const float ti = p.base + G * (p.per_k + p.per_round * R + p.per_load * (float(nb) / float(cus))) + p.round * R;
-        if (i == 0 || ti < t) {
+        const float t = p.t.us(a.K / QGROUP, float(nb) / float(cus), float((nb + cus - 1) / cus));
+        if (t < large_us) {
             best = i;
-            t = ti;
+            large_us = t;
         }
     }
     switch (best) {
